@@ -181,60 +181,101 @@ __global__ __launch_bounds__(kInstSpotThreads) void rt_batch_spots_kernel(const 
     }
 }
 
-constexpr int kSpotRays = 8;             // rays of one group per thread in stage 1
+// Group spots of stored rays in two launches: moments of (chunk, group), then
+// rt_spots_rows_kernel over each group's chunks.
+//
+// A workgroup of 256 lanes covers W = min(G, 256) consecutive groups and R =
+// 256 / W strides of the groups side by side (lane t: stride t / W, group
+// t % W), so its lanes read consecutive rays whatever G is; it walks its
+// chunk of S strides kSpotRays rays a lane at a time, held in registers: sum
+// and mean, then squared deviations (one division per kSpotRays rays), merged
+// across the passes and, in LDS by a fixed tree, across the lanes of a group.
+// One row per (chunk, group) leaves, group-major.  Bound by the row reads (17
+// bytes a ray) and, for small inputs, by the two launches.  One thread per 8
+// rays of a group (Welford, two divisions a ray, 40 bytes of partial per 8
+// rays) and one workgroup merging all of a group's partials took 7.4 + 27.9
+// us for 5e5 rays in 5 groups; this takes 6.0 + 4.4 (5e6 rays in one group:
+// 19.4 + 5.1, 4.4 TB/s).
+constexpr int kSpotThreads = 256;
+constexpr int kSpotRays = 8;             // rays of one group per lane and pass
 
-// stage 1: thread (chunk b, group g) takes the group's kSpotRays rays of the
-// chunk in order (Welford); consecutive threads read consecutive rays
-__global__ void rt_group_moments_kernel(const double* X, const double* Y, const signed char* F, uint64_t n,
-                                        uint64_t G, uint64_t n_chunks, double* part) {
-    const uint64_t idx = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= n_chunks * G) return;
-    const uint64_t b = idx / G, g = idx - b * G;
-    Mom m{0.0, 0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int k = 0; k < kSpotRays; ++k) {
-        const uint64_t r = (b * kSpotRays + k) * G + g;
-        if (r < n && F[r] == 1) {
-            const double x = X[r], y = Y[r];
-            m.n += 1.0;
-            const double dx = x - m.mx, dy = y - m.my;
-            m.mx += dx / m.n;
-            m.my += dy / m.n;
-            m.qx += dx * (x - m.mx);
-            m.qy += dy * (y - m.my);
-        }
-    }
-    double* o = part + idx * 5;
-    o[0] = m.n; o[1] = m.mx; o[2] = m.my; o[3] = m.qx; o[4] = m.qy;
+// strides of the groups per chunk: one pass of the workgroup, more passes
+// above 2^21 rays so that a group's merge has about 1,000 rows at most (the
+// rows of 1e7 rays in one group: 4,900 at one pass per chunk, 980 at five)
+__host__ __device__ inline uint64_t spot_chunk_strides(uint64_t n, uint64_t G) {
+    const uint64_t rows = G < (uint64_t)kSpotThreads ? kSpotThreads / G : 1;
+    return rows * kSpotRays * (1 + (n >> 21));
 }
 
-// stage 2: one workgroup per group; thread t merges chunks t, t + 256, ... in
-// order, then a fixed tree over the threads
-__global__ __launch_bounds__(256) void rt_group_spots_kernel(const double* part, uint64_t n_chunks, uint64_t G,
-                                                             double* spots) {
-    __shared__ Mom s[256];
-    const uint64_t g = blockIdx.x;
+// chunks of n rays in G groups (one, empty, for no rays)
+__host__ __device__ inline uint64_t spot_chunk_count(uint64_t n, uint64_t G) {
+    const uint64_t strides = (n + G - 1) / G, S = spot_chunk_strides(n, G);
+    return strides > 0 ? (strides + S - 1) / S : 1;
+}
+
+// the moments of chunk b of n rays (X, Y, F: the first ray's) for groups g0 ..
+// g0 + 255, to rows part[(g * n_rows + row) * 5 ..]
+__device__ __forceinline__ void group_moments_chunk(const double* X, const double* Y, const signed char* F, uint64_t n,
+                                                    uint64_t G, uint64_t b, uint64_t g0, double* part, uint64_t n_rows,
+                                                    uint64_t row) {
+    __shared__ Mom s[kSpotThreads];
+    const unsigned W = G < (uint64_t)kSpotThreads ? (unsigned)G : (unsigned)kSpotThreads, R = kSpotThreads / W;
+    const unsigned lane_row = threadIdx.x / W;
+    const uint64_t g = g0 + (threadIdx.x - lane_row * W);
+    const uint64_t S = spot_chunk_strides(n, G), s0 = b * S;
+    const bool on = lane_row < R && g < G;
     Mom m{0.0, 0.0, 0.0, 0.0, 0.0};
-    for (uint64_t b = threadIdx.x; b < n_chunks; b += 256) {
-        const double* o = part + (b * G + g) * 5;
-        m = mom_merge(m, Mom{o[0], o[1], o[2], o[3], o[4]});
+    for (uint64_t p = 0; p < S; p += (uint64_t)R * kSpotRays) {
+        double x[kSpotRays], y[kSpotRays];
+        bool live[kSpotRays];
+#pragma unroll
+        for (int k = 0; k < kSpotRays; ++k) {
+            const uint64_t r = (s0 + p + lane_row + (uint64_t)k * R) * G + g;
+            live[k] = on && r < n && F[r] == 1;
+            x[k] = live[k] ? X[r] : 0.0;
+            y[k] = live[k] ? Y[r] : 0.0;
+        }
+        Mom q{0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int k = 0; k < kSpotRays; ++k) {
+            q.n += live[k] ? 1.0 : 0.0;
+            q.mx += x[k];
+            q.my += y[k];
+        }
+        if (q.n > 0.0) {
+            q.mx /= q.n;
+            q.my /= q.n;
+#pragma unroll
+            for (int k = 0; k < kSpotRays; ++k) {
+                const double dx = live[k] ? x[k] - q.mx : 0.0, dy = live[k] ? y[k] - q.my : 0.0;
+                q.qx += dx * dx;
+                q.qy += dy * dy;
+            }
+        }
+        m = mom_merge(m, q);
     }
     s[threadIdx.x] = m;
     __syncthreads();
-    for (int k = 128; k > 0; k >>= 1) {
-        if ((int)threadIdx.x < k) s[threadIdx.x] = mom_merge(s[threadIdx.x], s[threadIdx.x + k]);
+    for (unsigned k = kSpotThreads / 2; k > 0; k >>= 1) {
+        if (lane_row < k && lane_row + k < R) s[threadIdx.x] = mom_merge(s[threadIdx.x], s[threadIdx.x + k * W]);
         __syncthreads();
     }
-    if (threadIdx.x == 0) {
-        const Mom r = s[0];
-        double* out = spots + g * RT_SPOT_STRIDE;
-        out[0] = r.n;
-        out[1] = r.mx;
-        out[2] = r.my;
-        out[3] = r.n > 0.0 ? r.qx / r.n : 0.0;
-        out[4] = r.n > 0.0 ? r.qy / r.n : 0.0;
-        out[5] = r.n > 0.0 ? sqrt((r.qx + r.qy) / r.n) : 0.0;
+    if (lane_row == 0 && on) {
+        const Mom r = s[threadIdx.x];
+        double* o = part + (g * n_rows + row) * 5;
+        o[0] = r.n; o[1] = r.mx; o[2] = r.my; o[3] = r.qx; o[4] = r.qy;
     }
+}
+
+// blocks of 256 groups, a workgroup each per chunk
+inline uint64_t spot_group_blocks(uint64_t G) { return (G + kSpotThreads - 1) / kSpotThreads; }
+
+// workgroup blockIdx.x = chunk x (blocks of 256 groups)
+__global__ __launch_bounds__(kSpotThreads) void rt_group_moments_kernel(const double* X, const double* Y,
+                                                                        const signed char* F, uint64_t n, uint64_t G,
+                                                                        uint64_t n_chunks, double* part) {
+    const uint64_t gb = blockIdx.x / n_chunks, b = blockIdx.x - gb * n_chunks;
+    group_moments_chunk(X, Y, F, n, G, b, gb * kSpotThreads, part, n_chunks, b);
 }
 
 // Spots from group-major partial rows (the traces' tile partials,
@@ -287,9 +328,8 @@ __global__ __launch_bounds__(NT) void rt_spots_rows_kernel(const double* part, u
 }
 
 // Batched spots: instance i's rays are [ray_start[i], ray_start[i+1]) of the
-// concatenated beam and ray r of the instance is in group r mod G.  Chunks of
-// kSpotRays group strides per instance, chunk_start the prefix over
-// instances (one thread, in order).
+// concatenated beam and ray r of the instance is in group r mod G.  Chunks as
+// for that instance's rays alone, chunk_start the prefix over instances.
 __global__ __launch_bounds__(1024) void rt_batch_chunks_kernel(const uint64_t* ray_start, uint64_t n_inst,
                                                                uint64_t G, uint64_t* chunk_start) {
     // one workgroup: chunk counts of 1024 instances at a time, an inclusive
@@ -299,13 +339,7 @@ __global__ __launch_bounds__(1024) void rt_batch_chunks_kernel(const uint64_t* r
     if (threadIdx.x == 0) chunk_start[0] = 0;
     for (uint64_t base = 0; base < n_inst; base += 1024) {
         const uint64_t i = base + threadIdx.x;
-        uint64_t v = 0;
-        if (i < n_inst) {
-            const uint64_t n = ray_start[i + 1] - ray_start[i];
-            const uint64_t strides = (n + G - 1) / G;
-            v = strides > 0 ? (strides + kSpotRays - 1) / kSpotRays : 1;
-        }
-        sc[threadIdx.x] = v;
+        sc[threadIdx.x] = i < n_inst ? spot_chunk_count(ray_start[i + 1] - ray_start[i], G) : 0;
         __syncthreads();
         for (int off = 1; off < 1024; off <<= 1) {
             const uint64_t add = (int)threadIdx.x >= off ? sc[threadIdx.x - off] : 0;
@@ -319,65 +353,22 @@ __global__ __launch_bounds__(1024) void rt_batch_chunks_kernel(const uint64_t* r
     }
 }
 
-__global__ void rt_batch_moments_kernel(const double* X, const double* Y, const signed char* F,
-                                        const uint64_t* ray_start, const uint64_t* chunk_start, uint64_t n_inst,
-                                        uint64_t G, double* part) {
-    const uint64_t idx = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const uint64_t total = chunk_start[n_inst];
-    if (idx >= total * G) return;
-    const uint64_t c = idx / G, g = idx - c * G;
+// workgroup blockIdx.x = chunk of the batch x (blocks of 256 groups); the
+// chunk's instance from the prefix
+__global__ __launch_bounds__(kSpotThreads) void rt_batch_moments_kernel(const double* X, const double* Y,
+                                                                        const signed char* F,
+                                                                        const uint64_t* ray_start,
+                                                                        const uint64_t* chunk_start, uint64_t n_inst,
+                                                                        uint64_t G, uint64_t n_chunks, double* part) {
+    const uint64_t gb = blockIdx.x / n_chunks, c = blockIdx.x - gb * n_chunks;
     uint64_t lo = 0, hi = n_inst;
     while (hi - lo > 1) {
         const uint64_t mid = (lo + hi) >> 1;
         if (chunk_start[mid] <= c) lo = mid; else hi = mid;
     }
-    const uint64_t r0 = ray_start[lo], n = ray_start[lo + 1] - r0, lc = c - chunk_start[lo];
-    Mom m{0.0, 0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int k = 0; k < kSpotRays; ++k) {
-        const uint64_t r = (lc * kSpotRays + k) * G + g;
-        if (r < n && F[r0 + r] == 1) {
-            const double x = X[r0 + r], y = Y[r0 + r];
-            m.n += 1.0;
-            const double dx = x - m.mx, dy = y - m.my;
-            m.mx += dx / m.n;
-            m.my += dy / m.n;
-            m.qx += dx * (x - m.mx);
-            m.qy += dy * (y - m.my);
-        }
-    }
-    double* o = part + idx * 5;
-    o[0] = m.n; o[1] = m.mx; o[2] = m.my; o[3] = m.qx; o[4] = m.qy;
-}
-
-// one workgroup per (instance, group) = blockIdx.x; the same merge order as
-// rt_group_spots_kernel over the instance's chunks
-__global__ __launch_bounds__(256) void rt_batch_spots_groups_kernel(const double* part, const uint64_t* chunk_start,
-                                                                    uint64_t G, double* spots) {
-    __shared__ Mom s[256];
-    const uint64_t ig = blockIdx.x, i = ig / G, g = ig - i * G;
-    const uint64_t c0 = chunk_start[i], nc = chunk_start[i + 1] - c0;
-    Mom m{0.0, 0.0, 0.0, 0.0, 0.0};
-    for (uint64_t b = threadIdx.x; b < nc; b += 256) {
-        const double* o = part + ((c0 + b) * G + g) * 5;
-        m = mom_merge(m, Mom{o[0], o[1], o[2], o[3], o[4]});
-    }
-    s[threadIdx.x] = m;
-    __syncthreads();
-    for (int k = 128; k > 0; k >>= 1) {
-        if ((int)threadIdx.x < k) s[threadIdx.x] = mom_merge(s[threadIdx.x], s[threadIdx.x + k]);
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        const Mom r = s[0];
-        double* out = spots + ig * RT_SPOT_STRIDE;
-        out[0] = r.n;
-        out[1] = r.mx;
-        out[2] = r.my;
-        out[3] = r.n > 0.0 ? r.qx / r.n : 0.0;
-        out[4] = r.n > 0.0 ? r.qy / r.n : 0.0;
-        out[5] = r.n > 0.0 ? sqrt((r.qx + r.qy) / r.n) : 0.0;
-    }
+    const uint64_t r0 = ray_start[lo];
+    group_moments_chunk(X + r0, Y + r0, F + r0, ray_start[lo + 1] - r0, G, c - chunk_start[lo], gb * kSpotThreads, part,
+                        n_chunks, c);
 }
 
 // One gradient-descent step on the device records of a batch: thread (i, s)
@@ -1896,23 +1887,26 @@ WorkBufs* thread_work(int dev) {
     return &g_thread_work.w;
 }
 
-int group_spots_launch(const double* X, const double* Y, const signed char* flag, uint64_t n, uint64_t G,
-                       uint64_t n_chunks, double* part, double* spots, hipStream_t st) {
+// moments of n rays in G groups (spot_chunk_count(n, G) rows of 5 doubles per
+// group in part), then the groups' spots
+int group_spots_launch(const double* X, const double* Y, const signed char* flag, uint64_t n, uint64_t G, double* part,
+                       double* spots, hipStream_t st) {
     // with n == 0 the single chunk is empty and its partials are written as zeros
-    const uint64_t threads = n_chunks * G;
-    hipLaunchKernelGGL(rt_group_moments_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, X, Y,
-                       flag, n, G, n_chunks, part);
+    const uint64_t n_chunks = spot_chunk_count(n, G);
+    hipLaunchKernelGGL(rt_group_moments_kernel, dim3((unsigned)(n_chunks * spot_group_blocks(G))), dim3(kSpotThreads),
+                       0, st, X, Y, flag, n, G, n_chunks, part);
     HIP_TRY(hipGetLastError(), RT_ERR_FAILED);
-    hipLaunchKernelGGL(rt_group_spots_kernel, dim3((unsigned)G), dim3(256), 0, st, (const double*)part, n_chunks,
-                       G, spots);
+    hipLaunchKernelGGL(rt_spots_rows_kernel<256>, dim3((unsigned)G), dim3(256), 0, st, (const double*)part, n_chunks,
+                       (const uint64_t*)nullptr, G, spots);
     HIP_TRY(hipGetLastError(), RT_ERR_FAILED);
     return RT_OK;
 }
 
-// chunks of kSpotRays strides of the groups over n rays
-uint64_t spot_chunks(uint64_t n, uint64_t G) {
+// partial moments of an input as the entry points' size limits count them:
+// one per 8 rays of a group
+uint64_t spot_partials(uint64_t n, uint64_t G) {
     const uint64_t strides = (n + G - 1) / G;
-    return strides > 0 ? (strides + kSpotRays - 1) / kSpotRays : 1;
+    return strides > 0 ? (strides + 7) / 8 : 1;
 }
 }  // namespace
 
@@ -1923,15 +1917,13 @@ extern "C" int rt_hip_group_spots(const double* X, const double* Y, const signed
     int rc = ensure_device();
     if (rc != RT_OK) return rc;
     const uint64_t G = n_groups;
-    const uint64_t n_chunks = spot_chunks(n, G);
-    if (n_chunks > (1ull << 40) / G) return set_error(RT_ERR_BAD_VALUE, "too many rays or groups");
+    if (spot_partials(n, G) > (1ull << 40) / G) return set_error(RT_ERR_BAD_VALUE, "too many rays or groups");
     int dev = 0;
     HIP_TRY(hipGetDevice(&dev), RT_ERR_FAILED);
     WorkBufs* w = thread_work(dev);
-    rc = w->ensure(WorkBufs::SPOT_PART, n_chunks * G * 5 * sizeof(double));
+    rc = w->ensure(WorkBufs::SPOT_PART, spot_chunk_count(n, G) * G * 5 * sizeof(double));
     if (rc != RT_OK) return rc;
-    return group_spots_launch(X, Y, flag, n, G, n_chunks, w->get<double>(WorkBufs::SPOT_PART), spots,
-                              (hipStream_t)stream);
+    return group_spots_launch(X, Y, flag, n, G, w->get<double>(WorkBufs::SPOT_PART), spots, (hipStream_t)stream);
 }
 
 // ------------------------------------ group spots without allocation
@@ -1981,12 +1973,12 @@ extern "C" int rt_hip_group_spots_noalloc(const double* X, const double* Y, cons
     if (n > 0 && (!X || !Y || !flag)) return set_error(RT_ERR_BAD_VALUE, "NULL ray array");
     const uint64_t G = n_groups;
     const uint64_t cap = kScratchDoubles / 5;                 // partial moments that fit
-    const uint64_t n_chunks = G <= cap ? spot_chunks(n, G) : 0;
-    if (G > cap || n_chunks > cap / G)
+    const uint64_t n_part = G <= cap ? spot_partials(n, G) : 0;
+    if (G > cap || n_part > cap / G)
         return set_error(RT_ERR_BAD_VALUE,
                          "%zu rays in %zu groups need %llu partial moments; the no-allocation entry point "
                          "holds %llu (use rt_hip_group_spots)",
-                         n, n_groups, (unsigned long long)(G > cap ? G : n_chunks * G), (unsigned long long)cap);
+                         n, n_groups, (unsigned long long)(G > cap ? G : n_part * G), (unsigned long long)cap);
     int rc = ensure_device();
     if (rc != RT_OK) return rc;
     int dev = 0;
@@ -1994,7 +1986,7 @@ extern "C" int rt_hip_group_spots_noalloc(const double* X, const double* Y, cons
     double* part = nullptr;
     rc = scratch_ptr(dev, &part);
     if (rc != RT_OK) return rc;
-    return group_spots_launch(X, Y, flag, n, G, n_chunks, part, spots, (hipStream_t)stream);
+    return group_spots_launch(X, Y, flag, n, G, part, spots, (hipStream_t)stream);
 }
 
 extern "C" int rt_hip_spot_loss(const double* spots, size_t n_groups, const double* target, double weight,
@@ -2021,10 +2013,7 @@ extern "C" int rt_hip_batch_group_spots(const rt_hip_batch* b, const double* X, 
     hipStream_t st = (hipStream_t)stream;
     const uint64_t G = n_groups;
     uint64_t chunks = 0;                 // the same count the device prefix forms
-    for (int i = 0; i < b->n_inst; ++i) {
-        const uint64_t n = b->ray_start[i + 1] - b->ray_start[i], strides = (n + G - 1) / G;
-        chunks += strides > 0 ? (strides + kSpotRays - 1) / kSpotRays : 1;
-    }
+    for (int i = 0; i < b->n_inst; ++i) chunks += spot_chunk_count(b->ray_start[i + 1] - b->ray_start[i], G);
     // the batch's own working memory (calls on one batch are stream-ordered)
     rc = b->work.ensure(WorkBufs::SPOT_PART, chunks * G * 5 * sizeof(double));
     if (rc == RT_OK) rc = b->work.ensure(WorkBufs::SPOT_CS, ((size_t)b->n_inst + 1) * sizeof(uint64_t));
@@ -2034,12 +2023,12 @@ extern "C" int rt_hip_batch_group_spots(const rt_hip_batch* b, const double* X, 
     hipLaunchKernelGGL(rt_batch_chunks_kernel, dim3(1), dim3(1024), 0, st, (const uint64_t*)b->ray_start_dev,
                        (uint64_t)b->n_inst, G, buf.cs);
     HIP_TRY(hipGetLastError(), RT_ERR_FAILED);
-    const uint64_t threads = chunks * G;
-    hipLaunchKernelGGL(rt_batch_moments_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, X, Y, flag,
-                       (const uint64_t*)b->ray_start_dev, (const uint64_t*)buf.cs, (uint64_t)b->n_inst, G, buf.part);
+    hipLaunchKernelGGL(rt_batch_moments_kernel, dim3((unsigned)(chunks * spot_group_blocks(G))), dim3(kSpotThreads), 0, st,
+                       X, Y, flag, (const uint64_t*)b->ray_start_dev, (const uint64_t*)buf.cs, (uint64_t)b->n_inst, G,
+                       chunks, buf.part);
     HIP_TRY(hipGetLastError(), RT_ERR_FAILED);
-    hipLaunchKernelGGL(rt_batch_spots_groups_kernel, dim3((unsigned)(b->n_inst * G)), dim3(256), 0, st,
-                       (const double*)buf.part, (const uint64_t*)buf.cs, G, spots);
+    hipLaunchKernelGGL(rt_spots_rows_kernel<256>, dim3((unsigned)(b->n_inst * G)), dim3(256), 0, st,
+                       (const double*)buf.part, chunks, (const uint64_t*)buf.cs, G, spots);
     HIP_TRY(hipGetLastError(), RT_ERR_FAILED);
     return RT_OK;
 }
