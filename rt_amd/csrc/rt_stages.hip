@@ -29,7 +29,6 @@ enum StageOp { OP_TRANSFORM, OP_NORMALIZE, OP_INTERSECT, OP_MASK, OP_REFLECT, OP
 struct StageArgs {
     double rec[rt::DEV_STRIDE];        // device record of the surface (first: kernarg offset 0)
     uint64_t n;
-    int op, pad;
     double *X, *Y, *Z, *cX, *cY, *cZ;
     const double* mu;                  // per-ray n1/n2 (refraction, transmissive gratings)
     const double* L;                   // per-ray m lambda / n2 / d (gratings)
@@ -45,7 +44,7 @@ __device__ __forceinline__ cptr kernarg_record() {
 // Adds v summed over the workgroup into *dst with one atomic (none for a
 // zero sum).  Every thread of the workgroup calls it, after its ray loop.
 __device__ void block_add(unsigned long long* dst, unsigned long long v) {
-    __shared__ unsigned long long part[kThreads / 64];
+    __shared__ unsigned long long part[16];              // waves of a workgroup, 1024 lanes at most
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
     if (__lane_id() == 0) part[threadIdx.x / 64] = v;
     __syncthreads();
@@ -57,53 +56,109 @@ __device__ void block_add(unsigned long long* dst, unsigned long long v) {
     __syncthreads();
 }
 
-__global__ __launch_bounds__(kThreads) void rt_stage_kernel(StageArgs a) {
+// The stages, one kernel each (a switch over all of them in one kernel held
+// the registers of the largest and loaded every array in every stage).  Bound
+// by the rows they read and write; a row that a stage's uniform structure
+// leaves alone is neither read nor written: a frame change without rotation
+// touches only the shifted coordinates (a translation along the axis, the
+// usual one between lens surfaces, 16 bytes a ray instead of 96: 15.2 -> 5.5
+// us at 1e6 rays), a plane surface's action needs no position.
+//
+// Atomics on one address are served one after the other, about 7-10 ns each,
+// so the stages that count add per workgroup, at most kCountBlocks of them (a
+// mask that loses rays in every wave: 113 -> 11 us at 1e6 rays with an add per
+// wave before; a Newton intersection 53 -> 20 us with one per 256 rays).
+constexpr int kCountThreads = 1024;
+constexpr unsigned kCountBlocks = 512;
+
+// frame change: which coordinates move (the same for every ray)
+struct Touch {
+    bool X, Y, Z, c[3];
+};
+template <class SD>
+__device__ __forceinline__ Touch transform_touch(const SD& d) {
+    const bool r0 = d.rot(0), r1 = d.rot(1), r2 = d.rot(2);
+    return Touch{r0 || r2 || d.p[RT_S_DIST + 0] != 0.0, r1 || r2 || d.p[RT_S_DIST + 1] != 0.0,
+                 r0 || r1 || d.p[RT_S_DIST + 2] != 0.0, {r0 || r2, r1 || r2, r0 || r1}};
+}
+
+__global__ __launch_bounds__(kThreads) void rt_transform_kernel(StageArgs a) {     // beam_transform, beam.cu:416-579
     const rt::DynSurf d{kernarg_record()};
+    const Touch t = transform_touch(d);
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    unsigned long long it_sum = 0;
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += stride) {
         Ray r;
-        r.X = a.X ? a.X[i] : 0.0; r.Y = a.Y ? a.Y[i] : 0.0; r.Z = a.Z ? a.Z[i] : 0.0;
-        r.cX = a.cX[i]; r.cY = a.cY[i]; r.cZ = a.cZ[i];
+        r.X = t.X ? a.X[i] : 0.0; r.Y = t.Y ? a.Y[i] : 0.0; r.Z = t.Z ? a.Z[i] : 0.0;
+        r.cX = t.c[0] ? a.cX[i] : 0.0; r.cY = t.c[1] ? a.cY[i] : 0.0; r.cZ = t.c[2] ? a.cZ[i] : 0.0;
+        rt::transform_ray(d, r);
+        if (t.X) a.X[i] = r.X;
+        if (t.Y) a.Y[i] = r.Y;
+        if (t.Z) a.Z[i] = r.Z;
+        if (t.c[0]) a.cX[i] = r.cX;
+        if (t.c[1]) a.cY[i] = r.cY;
+        if (t.c[2]) a.cZ[i] = r.cZ;
+    }
+}
+
+__global__ __launch_bounds__(kThreads) void rt_normalize_kernel(StageArgs a) {     // Beam::Normalize, beam.cpp:527-571
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += stride) {
+        double cX = a.cX[i], cY = a.cY[i], cZ = a.cZ[i];
+        rt::normalize_ray(cX, cY, cZ);
+        a.cX[i] = cX; a.cY[i] = cY; a.cZ[i] = cZ;
+    }
+}
+
+__global__ __launch_bounds__(kThreads) void rt_reflect_kernel(StageArgs a) {       // surface_reflection, surface.cu:883-951
+    const rt::DynSurf d{kernarg_record()};
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += stride) {
+        if (d.cls() == RT_PLANE) {
+            a.cZ[i] = -a.cZ[i];
+            continue;
+        }
+        Ray r{a.X[i], a.Y[i], a.Z[i], a.cX[i], a.cY[i], a.cZ[i], 0.0};
+        rt::reflect_ray(d, r);
+        a.cX[i] = r.cX; a.cY[i] = r.cY; a.cZ[i] = r.cZ;
+    }
+}
+
+// The counting stages.  OP_INTERSECT: surface_intersection (surface.cu:655-760);
+// OP_MASK: Surface/Shade::ApplyConstrains (surface.cpp:264-321, 652-699);
+// OP_REFRACT: surface_refraction (surface.cu:1155-1242); OP_DIFFRACT:
+// surface_diffration (surface.cu:1655-1768).
+template <int OP>
+__global__ __launch_bounds__(kCountThreads) void rt_count_stage_kernel(StageArgs a) {
+    const rt::DynSurf d{kernarg_record()};
+    const bool pos = OP == OP_INTERSECT || OP == OP_MASK || d.cls() != RT_PLANE;
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    unsigned long long it_sum = 0, lost_sum = 0;
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += stride) {
+        Ray r;
+        r.X = pos ? a.X[i] : 0.0; r.Y = pos ? a.Y[i] : 0.0;
         r.lam = 0.0;
-        bool lost = false;
+        bool lost;
         unsigned it = 0;
-        switch (a.op) {
-            case OP_TRANSFORM:                 // beam_transform, beam.cu:416-579
-                rt::transform_ray(d, r);
-                a.X[i] = r.X; a.Y[i] = r.Y; a.Z[i] = r.Z;
-                a.cX[i] = r.cX; a.cY[i] = r.cY; a.cZ[i] = r.cZ;
-                break;
-            case OP_NORMALIZE:                 // Beam::Normalize, beam.cpp:527-571
-                rt::normalize_ray(r.cX, r.cY, r.cZ);
-                a.cX[i] = r.cX; a.cY[i] = r.cY; a.cZ[i] = r.cZ;
-                break;
-            case OP_INTERSECT:                 // surface_intersection, surface.cu:655-760
+        if constexpr (OP == OP_MASK) {
+            lost = !rt::mask_ray(d, r.X, r.Y);
+        } else {
+            r.Z = pos ? a.Z[i] : 0.0;
+            r.cX = a.cX[i]; r.cY = a.cY[i]; r.cZ = a.cZ[i];
+            if constexpr (OP == OP_INTERSECT) {
                 lost = !rt::intersect_ray(d, r, it);
                 a.X[i] = r.X; a.Y[i] = r.Y; a.Z[i] = r.Z;
-                break;
-            case OP_MASK:                      // Surface/Shade::ApplyConstrains, surface.cpp:264-321,652-699
-                lost = !rt::mask_ray(d, r.X, r.Y);
-                break;
-            case OP_REFLECT:                   // surface_reflection, surface.cu:883-951
-                rt::reflect_ray(d, r);
-                a.cX[i] = r.cX; a.cY[i] = r.cY; a.cZ[i] = r.cZ;
-                break;
-            case OP_REFRACT:                   // surface_refraction, surface.cu:1155-1242
-                lost = !rt::refract_ray(d, r, a.mu[i]);
+            } else {
+                lost = OP == OP_REFRACT ? !rt::refract_ray(d, r, a.mu[i])
+                                        : !rt::diffract_ray(d, r, a.mu ? a.mu[i] : 1.0, a.L[i]);
                 if (!lost) { a.cX[i] = r.cX; a.cY[i] = r.cY; a.cZ[i] = r.cZ; }
-                break;
-            case OP_DIFFRACT:                  // surface_diffration, surface.cu:1655-1768
-                lost = !rt::diffract_ray(d, r, a.mu ? a.mu[i] : 1.0, a.L[i]);
-                if (!lost) { a.cX[i] = r.cX; a.cY[i] = r.cY; a.cZ[i] = r.cZ; }
-                break;
+            }
         }
         if (lost) a.flag[i] = 0;
-        unsigned long long b = __ballot(lost);
-        if (__lane_id() == 0 && b && a.n_bad) atomicAdd(a.n_bad, (unsigned long long)__popcll(b));
+        lost_sum += lost ? 1 : 0;
         it_sum += it;
     }
-    if (a.iters) block_add(a.iters, it_sum);
+    if (a.n_bad) block_add(a.n_bad, lost_sum);
+    if (OP == OP_INTERSECT && a.iters) block_add(a.iters, it_sum);
 }
 
 enum BeamOp { GEN_POSITIONS, GEN_DIRECTIONS, GEN_WAVELENGTHS };
@@ -148,27 +203,30 @@ struct CcdArgs {
     double* image;
     unsigned* hist;
     unsigned long long* offchip;
-    int op;
 };
 
-// ccd_coordinates_kernel (rt_cuda_engine_ccd.cu:30-45) and
-// compute_ccd_image_kernel (:219-232) with atomics and a bounds check (D10)
-__global__ __launch_bounds__(kThreads) void rt_ccd_kernel(CcdArgs a) {
+// ccd_coordinates_kernel (rt_cuda_engine_ccd.cu:30-45)
+__global__ __launch_bounds__(kThreads) void rt_ccd_coordinates_kernel(CcdArgs a) {
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += stride) {
-        if (a.op == 0) {
-            a.ccdX[i] = rt::trunc_u32((a.X[i] + a.half_x) / a.xpix);
-            a.ccdY[i] = rt::trunc_u32((a.Y[i] + a.half_y) / a.ypix);
-        } else {
-            uint32_t px = a.ccdX[i], py = a.ccdY[i];
-            bool off = !(px < a.xdim && py < a.ydim);
-            uint32_t pix = off ? 0u : py * a.xdim + px;     // xdim * ydim <= 2^32 (checked on the host)
-            if (!off && a.image) unsafeAtomicAdd(&a.image[pix], a.w ? a.w[i] : 1.0);
-            if (a.hist) rt::hist_add_wave(a.hist, pix, !off);
-            unsigned long long b = __ballot(off);
-            if (__lane_id() == 0 && b && a.offchip) atomicAdd(a.offchip, (unsigned long long)__popcll(b));
-        }
+        a.ccdX[i] = rt::trunc_u32((a.X[i] + a.half_x) / a.xpix);
+        a.ccdY[i] = rt::trunc_u32((a.Y[i] + a.half_y) / a.ypix);
     }
+}
+
+// compute_ccd_image_kernel (ccd.cu:219-232) with atomics and a bounds check (D10)
+__global__ __launch_bounds__(kCountThreads) void rt_ccd_accumulate_kernel(CcdArgs a) {
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    unsigned long long off_sum = 0;
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += stride) {
+        uint32_t px = a.ccdX[i], py = a.ccdY[i];
+        bool off = !(px < a.xdim && py < a.ydim);
+        uint32_t pix = off ? 0u : py * a.xdim + px;     // xdim * ydim <= 2^32 (checked on the host)
+        if (!off && a.image) unsafeAtomicAdd(&a.image[pix], a.w ? a.w[i] : 1.0);
+        if (a.hist) rt::hist_add_wave(a.hist, pix, !off);
+        off_sum += off ? 1 : 0;
+    }
+    if (a.offchip) block_add(a.offchip, off_sum);
 }
 
 struct ScaleArgs {
@@ -236,20 +294,27 @@ __global__ __launch_bounds__(kThreads) void rt_spline_kernel(SplineArgs a) {
     extern __shared__ double s_sp[];
     for (int i = threadIdx.x; i < a.pool_len; i += blockDim.x) s_sp[i] = a.spline[i];
     __syncthreads();
+    unsigned long long oob_sum = 0;
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += stride) {
         int err = 0;
         double v = rt::spline_eval(s_sp, a.x[i], err);
         a.y[i] = err ? 0.0 : v;
-        unsigned long long b = __ballot(err != 0);
-        if (__lane_id() == 0 && b && a.oob) atomicAdd(a.oob, (unsigned long long)__popcll(b));
+        oob_sum += err != 0 ? 1 : 0;
     }
+    if (a.oob) block_add(a.oob, oob_sum);
 }
 
 unsigned grid_for(size_t n) {
     uint64_t want = (n + kThreads - 1) / kThreads;
     uint64_t cap = (uint64_t)rt_device_cus() * 16;
     return (unsigned)(want < cap ? (want ? want : 1) : cap);
+}
+
+// workgroups of kCountThreads lanes of a counting kernel
+unsigned count_grid(size_t n) {
+    const uint64_t want = (n + kCountThreads - 1) / kCountThreads;
+    return (unsigned)(want < kCountBlocks ? (want ? want : 1) : kCountBlocks);
 }
 
 int launch_stage(const double* rec, size_t n, int op, double* X, double* Y, double* Z, double* cX, double* cY,
@@ -261,10 +326,19 @@ int launch_stage(const double* rec, size_t n, int op, double* X, double* Y, doub
     StageArgs a;
     memset(&a, 0, sizeof a);
     if (rec) rt_device_record(rec, a.rec);
-    a.n = n; a.op = op;
+    a.n = n;
     a.X = X; a.Y = Y; a.Z = Z; a.cX = cX; a.cY = cY; a.cZ = cZ;
     a.mu = mu; a.L = L; a.flag = flag; a.n_bad = n_bad; a.iters = iters;
-    hipLaunchKernelGGL(rt_stage_kernel, dim3(grid_for(n)), dim3(kThreads), 0, (hipStream_t)stream, a);
+    const bool count = op == OP_INTERSECT || op == OP_MASK || op == OP_REFRACT || op == OP_DIFFRACT;
+    auto kern = op == OP_TRANSFORM   ? rt_transform_kernel
+                : op == OP_NORMALIZE ? rt_normalize_kernel
+                : op == OP_INTERSECT ? rt_count_stage_kernel<OP_INTERSECT>
+                : op == OP_MASK      ? rt_count_stage_kernel<OP_MASK>
+                : op == OP_REFLECT   ? rt_reflect_kernel
+                : op == OP_REFRACT   ? rt_count_stage_kernel<OP_REFRACT>
+                                     : rt_count_stage_kernel<OP_DIFFRACT>;
+    hipLaunchKernelGGL(kern, dim3(count ? count_grid(n) : grid_for(n)), dim3(count ? kCountThreads : kThreads), 0,
+                       (hipStream_t)stream, a);
     HIP_TRY(hipGetLastError(), RT_ERR_FAILED);
     return RT_OK;
 }
@@ -313,8 +387,8 @@ extern "C" int rt_hip_stage_intersect(const double* rec, size_t n, double* X, do
 extern "C" int rt_hip_stage_mask(const double* rec, size_t n, double* X, double* Y, signed char* flag,
                                  unsigned long long* n_bad, void* stream) {
     if (!rec || !X || !Y || !flag) return rt_set_error(RT_ERR_BAD_VALUE, "NULL argument");
-    // the stage kernel reads direction cosines; give it the positions (unused by the mask)
-    return launch_stage(rec, n, OP_MASK, X, Y, nullptr, X, Y, X, nullptr, nullptr, flag, n_bad, nullptr, stream);
+    return launch_stage(rec, n, OP_MASK, X, Y, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, flag, n_bad, nullptr,
+                        stream);
 }
 
 extern "C" int rt_hip_stage_reflect(const double* rec, size_t n, double* X, double* Y, double* Z, double* cX,
@@ -396,8 +470,8 @@ extern "C" int rt_hip_ccd_coordinates(size_t n, const double* X, const double* Y
     CcdArgs a;
     memset(&a, 0, sizeof a);
     a.n = n; a.half_x = xsize / 2.0; a.half_y = ysize / 2.0; a.xpix = xpix; a.ypix = ypix;
-    a.X = X; a.Y = Y; a.ccdX = ccdX; a.ccdY = ccdY; a.op = 0;
-    hipLaunchKernelGGL(rt_ccd_kernel, dim3(grid_for(n)), dim3(kThreads), 0, (hipStream_t)stream, a);
+    a.X = X; a.Y = Y; a.ccdX = ccdX; a.ccdY = ccdY;
+    hipLaunchKernelGGL(rt_ccd_coordinates_kernel, dim3(grid_for(n)), dim3(kThreads), 0, (hipStream_t)stream, a);
     HIP_TRY(hipGetLastError(), RT_ERR_FAILED);
     return RT_OK;
 }
@@ -416,8 +490,8 @@ extern "C" int rt_hip_ccd_accumulate(size_t n, const unsigned* ccdX, const unsig
     memset(&a, 0, sizeof a);
     a.n = n; a.xdim = (uint32_t)xdim; a.ydim = (uint32_t)ydim;
     a.ccdX = (unsigned*)ccdX; a.ccdY = (unsigned*)ccdY; a.w = w; a.image = image; a.hist = hist;
-    a.offchip = offchip; a.op = 1;
-    hipLaunchKernelGGL(rt_ccd_kernel, dim3(grid_for(n)), dim3(kThreads), 0, (hipStream_t)stream, a);
+    a.offchip = offchip;
+    hipLaunchKernelGGL(rt_ccd_accumulate_kernel, dim3(count_grid(n)), dim3(kCountThreads), 0, (hipStream_t)stream, a);
     HIP_TRY(hipGetLastError(), RT_ERR_FAILED);
     return RT_OK;
 }

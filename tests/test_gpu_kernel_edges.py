@@ -41,3 +41,61 @@ def test_group_spots_at_chunk_edges(hip, n, G):
     # differences that carry 12.5 * 2^-53 each, against a variance of 1e-4
     assert np.all(np.abs(got[:, 1:3] - want[:, 1:3]) <= 1e-13)
     assert np.all(np.abs(got[:, 3:6] - want[:, 3:6]) <= 1e-10 * np.abs(want[:, 3:6]) + 1e-28)
+
+
+# one lane, one wave, a workgroup of the counting stages and its neighbours,
+# more rays than their largest grid holds at once
+@pytest.mark.parametrize("n", [1, 64, 1023, 1024, 1025, 512 * 1024 + 1])
+def test_mask_counts_and_flags(hip, n):
+    print(f"[mask] n={n}", flush=True)
+    from rt_amd import scheme as S
+    g = torch.Generator().manual_seed(n)
+    xy = torch.randn((2, n), generator=g, dtype=torch.float64)
+    if n > 64:
+        xy[0, 5], xy[1, 7] = float("nan"), float("inf")
+    rec = S.Scheme([S.Surface(S.RT_PLANE, S.RT_MIRROR, S.RT_CIRCLE, size=(1.25, 0.0), center=(0.1, -0.2))],
+                   S.Beam()).table
+    dev, flag = xy.cuda(), torch.ones(n, dtype=torch.int8, device="cuda")
+    bad = torch.full((2,), 3, dtype=torch.int64, device="cuda")
+    hip.check(hip.lib().rt_hip_stage_mask(hip._dptr(np.ascontiguousarray(rec)), n, dev[0].data_ptr(), dev[1].data_ptr(),
+                                          flag.data_ptr(), bad.data_ptr(), torch.cuda.current_stream().cuda_stream), "mask")
+    # the aperture rejects what compares outside it: a NaN stays
+    x, y = xy[0].numpy() - 0.1, xy[1].numpy() + 0.2
+    lost = x * x + y * y > 1.25 * 1.25
+    assert np.array_equal(flag.cpu().numpy() == 0, lost)
+    assert bad.cpu().tolist() == [3 + int(lost.sum()), 3]
+
+
+# every pattern of shifted coordinates and applied rotations: what moves moves
+# as in plain arithmetic, what the frame change leaves alone keeps its bits
+@pytest.mark.parametrize("dist", [(0.0, 0.0, 5.0), (1.5, 0.0, 0.0), (0.0, -2.0, 0.0), (0.3, 0.4, -7.0), (0.0, 0.0, 0.0)])
+@pytest.mark.parametrize("ang", [(0.0, 0.0, 0.0), (0.2, 0.0, 0.0), (0.0, -0.3, 0.0), (0.0, 0.0, 1.1), (0.1, 0.2, 0.3)])
+def test_transform_touches_what_it_moves(hip, dist, ang):
+    print(f"[transform] dist={dist} ang={ang}", flush=True)
+    n = 300
+    g = torch.Generator().manual_seed(1)
+    st = torch.randn((6, n), generator=g, dtype=torch.float64) * 50.0
+    st[0, 3], st[4, 9] = -0.0, float("nan")
+    dev = st.cuda()
+    ptr = [dev[k].data_ptr() for k in range(6)]
+    a, d = np.array(ang), np.array(dist)
+    hip.check(hip.lib().rt_hip_stage_transform(hip._dptr(a), hip._dptr(d), n, *ptr,
+                                               torch.cuda.current_stream().cuda_stream), "transform")
+    want, moved = st.numpy().copy(), [False] * 6
+    for k in range(3):
+        want[k] -= dist[k]
+        moved[k] = dist[k] != 0.0
+    for k, (u, v) in enumerate(((0, 2), (1, 2), (0, 1))):
+        if ang[k] == 0.0:
+            continue
+        s, c = np.sin(ang[k]), np.cos(ang[k])
+        for w in (0, 3):
+            want[u + w], want[v + w] = want[u + w] * c - want[v + w] * s, want[u + w] * s + want[v + w] * c
+            moved[u + w] = moved[v + w] = True
+    got = dev.cpu().numpy()
+    for k in range(6):
+        if not moved[k]:
+            assert got[k].tobytes() == st[k].numpy().tobytes(), k
+        else:
+            # up to three rotations of values near 150: a few units of 150 * 2^-53
+            assert np.allclose(got[k], want[k], rtol=0.0, atol=3e-13, equal_nan=True), k
