@@ -963,8 +963,8 @@ struct TraceArgs {
     // above for every instance)
     const double* inst_beams;
     // recording traces (kernels built with kRecLoss / kRecExt): the loss code
-    // of every ray, and the extents keys (n_surf x kExtPerSurf, ord_key
-    // encoded, combined with atomic min / max)
+    // of every ray, and every workgroup's extents keys (ext_add; key k of
+    // workgroup w at ext[k * workgroups + w])
     unsigned char* loss;
     unsigned long long* ext;
     // group spot partials (kernels built with kRecSpots, and batched traces
@@ -1028,6 +1028,7 @@ struct TraceCtx {
     const double* pool;           // LDS copy
     unsigned* st;                 // per-block LDS counters (RT_STATS_LEN)
     unsigned long long* ext;      // per-block LDS extents keys (recording kernels)
+    double* ext_bnd;              // bounds those keys cover (ext_add)
     unsigned char loss;           // loss code of the current ray (recording kernels)
     unsigned* hist;
     double* flux;
@@ -1065,19 +1066,83 @@ __device__ __forceinline__ void hist_add_wave(unsigned* hist, uint32_t pix, bool
     if (mine) atomicAdd(&hist[pix], 1u);
 }
 
-// Extents: the wave's min and max of v over the lanes with `on`, folded into
-// the block's keys e[2 q] (min) and e[2 q + 1] (max).  Called by every lane
-// of the wave (converged code).
-__device__ __forceinline__ void ext_add(unsigned long long* e, int q, bool on, double v) {
-    double lo = on ? v : __builtin_inf(), hi = on ? v : -__builtin_inf();
-    for (int m = 32; m >= 1; m >>= 1) {
-        lo = fmin(lo, __shfl_xor(lo, m));
-        hi = fmax(hi, __shfl_xor(hi, m));
+// A double moved between lanes by a DPP pattern inside rows of 16 lanes
+// (every source lane active).
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double v) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)u, CTRL, 0xF, 0xF, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(u >> 32), CTRL, 0xF, 0xF, false);
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+
+// x and y exchanged by v_permlane16_swap (H = 16: odd rows of 16 lanes of x
+// with even rows of y) or v_permlane32_swap (H = 32: upper half of x with
+// lower half of y): the two results.
+template <int H>
+__device__ __forceinline__ void swap_f64(double& x, double& y) {
+    const uint64_t ux = __builtin_bit_cast(uint64_t, x), uy = __builtin_bit_cast(uint64_t, y);
+    uint32_t l0, l1, h0, h1;
+    if (H == 16) {
+        const auto a = __builtin_amdgcn_permlane16_swap((uint32_t)ux, (uint32_t)uy, false, false);
+        const auto b = __builtin_amdgcn_permlane16_swap((uint32_t)(ux >> 32), (uint32_t)(uy >> 32), false, false);
+        l0 = a[0]; l1 = a[1]; h0 = b[0]; h1 = b[1];
+    } else {
+        const auto a = __builtin_amdgcn_permlane32_swap((uint32_t)ux, (uint32_t)uy, false, false);
+        const auto b = __builtin_amdgcn_permlane32_swap((uint32_t)(ux >> 32), (uint32_t)(uy >> 32), false, false);
+        l0 = a[0]; l1 = a[1]; h0 = b[0]; h1 = b[1];
     }
-    const bool any = __ballot(on) != 0;
-    if (any && __lane_id() == 0) {
-        atomicMin(&e[2 * q], ord_key(lo));
-        atomicMax(&e[2 * q + 1], ord_key(hi));
+    x = __builtin_bit_cast(double, ((uint64_t)h0 << 32) | l0);
+    y = __builtin_bit_cast(double, ((uint64_t)h1 << 32) | l1);
+}
+
+// x and y exchanged as above and added: lanes of row pair (2k, 2k+1), or of
+// the two halves, get x's rows summed in the even row (half) and y's rows
+// summed in the odd one, the lower row's value first.
+template <int H>
+__device__ __forceinline__ double swap_sum(double x, double y) {
+    swap_f64<H>(x, y);
+    return x + y;
+}
+
+template <int H>
+__device__ __forceinline__ double swap_min(double x, double y) {
+    swap_f64<H>(x, y);
+    return fmin(x, y);
+}
+
+// Extents.  The block's keys e[0 .. 2 NV) (LDS) take the minimum of v and of
+// -v (so of -max v) of each of NV values over the lanes with `on`, as ord_key;
+// b holds bounds, in the same order, that the keys cover already.  Called by
+// every lane of the wave (converged code).  Over a workgroup's many rays a new
+// extreme is rare, so a wave whose values all lie inside the bounds is done
+// after an LDS read and a compare a bound; otherwise the wave's minima are
+// formed together, the values transposed into the rows of 16 lanes on the way
+// (two values: rows 0, 1, 2, 3 end with min x, min y, min -x, min -y), and the
+// first lane of each row adds its own.  Whatever waves overwrite in the bounds
+// is covered by the keys.  A NaN never lies inside and adds the empty interval.
+// Bound by the instructions of the slow path in a workgroup's first rounds
+// (hence few, long-lived workgroups).  A reduction of every value for every
+// wave and atomics of every workgroup on the same 144 keys took 676 us for 2e6
+// rays of 12 surfaces, against 193 without extents; this takes 335.
+template <int NV>
+__device__ __forceinline__ void ext_add(unsigned long long* e, double* b, bool on, double x, double y = 0.0) {
+    bool inside = x >= b[0] && -x >= b[1];
+    if (NV == 2) inside = inside && y >= b[2] && -y >= b[3];
+    if (__ballot(on && !inside) == 0) return;
+    const double inf = __builtin_inf();
+    const bool xon = on && x == x, yon = on && y == y;
+    double t = swap_min<32>(xon ? x : inf, xon ? -x : inf);
+    t = swap_min<16>(t, NV == 2 ? swap_min<32>(yon ? y : inf, yon ? -y : inf) : t);
+    t = fmin(t, dpp_f64<0xB1>(t));
+    t = fmin(t, dpp_f64<0x4E>(t));
+    t = fmin(t, dpp_f64<0x141>(t));
+    t = fmin(t, dpp_f64<0x140>(t));
+    const unsigned lane = __lane_id(), row = lane >> 4;
+    const unsigned k = NV == 2 ? (row >> 1) | ((row & 1) << 1) : row >> 1;    // rows 0..3: x, y, -x, -y
+    if ((lane & 15) == 0 && (NV == 2 || (row & 1) == 0)) {
+        atomicMin(&e[k], ord_key(t));
+        if (t < b[k]) b[k] = t;
     }
 }
 
@@ -1110,7 +1175,7 @@ __device__ __forceinline__ void surface_step(const SD& d0, int s, Ray& r, bool& 
         // only the first surface and rotated frames normalise here
         if (s == 0 || d.rot(0) || d.rot(1) || d.rot(2)) normalize_ray(r.cX, r.cY, r.cZ);
     }
-    if constexpr ((MODE & kRecExt) != 0) ext_add(c.ext + s * kExtPerSurf, 0, alive, r.cZ);   // :995
+    if constexpr ((MODE & kRecExt) != 0) ext_add<1>(c.ext + s * kExtPerSurf, c.ext_bnd + s * kExtPerSurf, alive, r.cZ);   // :995
     if (d.type() == RT_AUXTYPE) return;                          // :1000
     unsigned long long entering = __ballot(alive);
     if (__lane_id() == 0 && entering) atomicAdd(&c.st[RT_ST_SURF + 4 * s], (unsigned)__popcll(entering));
@@ -1184,11 +1249,10 @@ __device__ __forceinline__ void surface_step(const SD& d0, int s, Ray& r, bool& 
         // the action changes only the cosines, so X, Y are still those of
         // the intersection (:1005-1008) and of the mask (:1017-1020)
         unsigned long long* e = c.ext + s * kExtPerSurf;
-        ext_add(e, 1, met, r.X);
-        ext_add(e, 2, met, r.Y);
-        ext_add(e, 3, passed, r.X);
-        ext_add(e, 4, passed, r.Y);
-        ext_add(e, 5, alive, r.cZ);                              // :1042
+        double* b = c.ext_bnd + s * kExtPerSurf;
+        ext_add<2>(e + 2, b + 2, met, r.X, r.Y);
+        ext_add<2>(e + 6, b + 6, passed, r.X, r.Y);
+        ext_add<1>(e + 10, b + 10, alive, r.cZ);                 // :1042
     }
     if constexpr ((MODE & kRecLoss) != 0) {
         if (lost_int) c.loss = (unsigned char)(1 + 3 * s);
@@ -1438,16 +1502,21 @@ __device__ __forceinline__ void trace_body(const TraceArgs& a, Surfaces surfaces
     extern __shared__ double s_pool[];
     __shared__ unsigned s_stats[RT_STATS_LEN];
     __shared__ unsigned long long s_ext[(MODE & kRecExt) ? RT_MAX_SURF * kExtPerSurf : 1];
+    __shared__ double s_bnd[(MODE & kRecExt) ? RT_MAX_SURF * kExtPerSurf : 1];
     for (int i = threadIdx.x; i < RT_STATS_LEN; i += blockDim.x) s_stats[i] = 0u;
     for (int i = threadIdx.x; i < a.pool_len; i += blockDim.x) s_pool[i] = a.pool[i];
     if constexpr ((MODE & kRecExt) != 0)
-        for (int i = threadIdx.x; i < RT_MAX_SURF * kExtPerSurf; i += blockDim.x) s_ext[i] = (i & 1) ? 0ull : ~0ull;
+        for (int i = threadIdx.x; i < RT_MAX_SURF * kExtPerSurf; i += blockDim.x) {
+            s_ext[i] = ~0ull;
+            s_bnd[i] = __builtin_inf();
+        }
     __syncthreads();
 
     TraceCtx c;
     c.pool = s_pool;
     c.st = s_stats;
     c.ext = s_ext;
+    c.ext_bnd = s_bnd;
     c.loss = 0;
     c.hist = a.hist;
     c.flux = a.flux;
@@ -1538,47 +1607,11 @@ __device__ __forceinline__ void trace_body(const TraceArgs& a, Surfaces surfaces
             if (s_stats[k]) atomicAdd(&dst[k], (unsigned long long)s_stats[k]);
     }
     if constexpr ((MODE & kRecExt) != 0) {
-        for (int k = threadIdx.x; k < a.n_surf * kExtPerSurf; k += blockDim.x) {
-            const unsigned long long v = s_ext[k];
-            if (k & 1) {
-                if (v != 0ull) atomicMax(&a.ext[k], v);
-            } else if (v != ~0ull) {
-                atomicMin(&a.ext[k], v);
-            }
-        }
+        // a row per workgroup, reduced afterwards (atomics of every workgroup on
+        // the same few lines are served one after the other)
+        for (int k = threadIdx.x; k < a.n_surf * kExtPerSurf; k += blockDim.x)
+            a.ext[(size_t)k * gridDim.x + blockIdx.x] = s_ext[k];
     }
-}
-
-// A double moved between lanes by a DPP pattern inside rows of 16 lanes
-// (every source lane active).
-template <int CTRL>
-__device__ __forceinline__ double dpp_f64(double v) {
-    const uint64_t u = __builtin_bit_cast(uint64_t, v);
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)u, CTRL, 0xF, 0xF, false);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(u >> 32), CTRL, 0xF, 0xF, false);
-    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
-}
-
-// x and y exchanged by v_permlane16_swap (H = 16: odd rows of 16 lanes of x
-// with even rows of y) or v_permlane32_swap (H = 32: upper half of x with
-// lower half of y), the two results added: lanes of row pair (2k, 2k+1), or of
-// the two halves, get x's rows summed in the even row (half) and y's rows
-// summed in the odd one, the lower row's value first.
-template <int H>
-__device__ __forceinline__ double swap_sum(double x, double y) {
-    const uint64_t ux = __builtin_bit_cast(uint64_t, x), uy = __builtin_bit_cast(uint64_t, y);
-    uint32_t l0, l1, h0, h1;
-    if (H == 16) {
-        const auto a = __builtin_amdgcn_permlane16_swap((uint32_t)ux, (uint32_t)uy, false, false);
-        const auto b = __builtin_amdgcn_permlane16_swap((uint32_t)(ux >> 32), (uint32_t)(uy >> 32), false, false);
-        l0 = a[0]; l1 = a[1]; h0 = b[0]; h1 = b[1];
-    } else {
-        const auto a = __builtin_amdgcn_permlane32_swap((uint32_t)ux, (uint32_t)uy, false, false);
-        const auto b = __builtin_amdgcn_permlane32_swap((uint32_t)(ux >> 32), (uint32_t)(uy >> 32), false, false);
-        l0 = a[0]; l1 = a[1]; h0 = b[0]; h1 = b[1];
-    }
-    return __builtin_bit_cast(double, ((uint64_t)h0 << 32) | l0) +
-           __builtin_bit_cast(double, ((uint64_t)h1 << 32) | l1);
 }
 
 // sum over the 16 lanes of each row (pairs, quads, 8, 16), the same value in

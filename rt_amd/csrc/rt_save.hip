@@ -42,26 +42,63 @@ __global__ void rt_save_zero_kernel(unsigned long long* v, int n) {
     for (int i = threadIdx.x; i < n; i += blockDim.x) v[i] = 0ull;
 }
 
-// counts of every loss code
-__global__ __launch_bounds__(256) void rt_loss_hist_kernel(const unsigned char* loss, uint64_t n,
-                                                           unsigned long long* counts) {
+// Position p holds ray p before the first stage, and the counts of every loss
+// code: one pass over the codes (1 byte read, 9 written a ray), V rays a lane
+// (V = 4 where the codes are 4-byte aligned).  Nearly every ray has code 0, so
+// those are counted in a register, the others in LDS; at most kInitBlocks
+// workgroups add to the counts, which share a few lines and are served one add
+// after the other.  (Two kernels, an LDS add per ray and 4,096 workgroups took
+// 52 + 7 us at 2e6 rays; this takes 13.5.)
+constexpr int kInitThreads = 512;
+constexpr unsigned kInitBlocks = 512;
+
+template <int V>
+__global__ __launch_bounds__(kInitThreads) void rt_order_init_kernel(const unsigned char* loss, uint64_t n,
+                                                                     uint64_t* perm, unsigned char* lpos,
+                                                                     unsigned long long* counts) {
     __shared__ unsigned h[256];
-    h[threadIdx.x] = 0u;
+    if (threadIdx.x < 256) h[threadIdx.x] = 0u;
     __syncthreads();
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
-        atomicAdd(&h[loss[i]], 1u);
+    unsigned good = 0;
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x * V;
+    for (uint64_t p = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) * V; p < n; p += stride) {
+        if (V == 4 && p + V <= n) {
+            const uint32_t c4 = *(const uint32_t*)(loss + p);
+            *(uint32_t*)(lpos + p) = c4;                 // (lpos: this library's own buffer, aligned)
+#pragma unroll
+            for (int k = 0; k < V; ++k) {
+                perm[p + k] = p + k;
+                const unsigned c = (c4 >> (8 * k)) & 255u;
+                if (c) atomicAdd(&h[c], 1u);
+                else ++good;
+            }
+        } else {
+            for (uint64_t q = p; q < n && q < p + V; ++q) {
+                const unsigned c = loss[q];
+                lpos[q] = (unsigned char)c;
+                perm[q] = q;
+                if (c) atomicAdd(&h[c], 1u);
+                else ++good;
+            }
+        }
+    }
+    for (int m = 32; m >= 1; m >>= 1) good += __shfl_xor(good, m);
+    if (__lane_id() == 0 && good) atomicAdd(&h[0], good);
     __syncthreads();
-    if (h[threadIdx.x]) atomicAdd(&counts[threadIdx.x], (unsigned long long)h[threadIdx.x]);
+    if (threadIdx.x < 256 && h[threadIdx.x]) atomicAdd(&counts[threadIdx.x], (unsigned long long)h[threadIdx.x]);
 }
 
-// position p holds ray p before the first stage
-__global__ void rt_order_init_kernel(const unsigned char* loss, uint64_t n, uint64_t* perm, unsigned char* lpos) {
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; p < n; p += stride) {
-        perm[p] = p;
-        lpos[p] = loss[p];
-    }
+// the 16 codes of a thread's positions base .. base + 15 (lpos is padded to a
+// whole tile), as bit k of a mask: position base + k is below G and has `code`
+__device__ __forceinline__ unsigned code_mask(const unsigned char* lpos, uint64_t base, uint64_t G,
+                                              unsigned char code) {
+    const uint4 v = *(const uint4*)(lpos + base);
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+    unsigned m = 0;
+#pragma unroll
+    for (int k = 0; k < kPerThread; ++k)
+        m |= (base + k < G && ((w[k / 4] >> (8 * (k % 4))) & 255u) == code) ? 1u << k : 0u;
+    return m;
 }
 
 // lost rays of this stage (code) per tile of [0, G)
@@ -69,11 +106,7 @@ __global__ __launch_bounds__(kTileThreads) void rt_stage_count_kernel(const unsi
                                                                       unsigned char code, uint64_t* tile_bad) {
     __shared__ unsigned s[kTileThreads / 64];
     const uint64_t base = (uint64_t)blockIdx.x * kTile + (uint64_t)threadIdx.x * kPerThread;
-    unsigned c = 0;
-    for (int k = 0; k < kPerThread; ++k) {
-        const uint64_t p = base + k;
-        c += (p < G && lpos[p] == code) ? 1u : 0u;
-    }
+    unsigned c = __popc(code_mask(lpos, base, G, code));
     for (int m = 32; m >= 1; m >>= 1) c += __shfl_xor(c, m);
     if (__lane_id() == 0) s[threadIdx.x / 64] = c;
     __syncthreads();
@@ -109,34 +142,25 @@ __global__ __launch_bounds__(1024) void rt_tile_scan_kernel(uint64_t* tile_bad, 
     }
 }
 
-// per position of tile `tile`: lost rays of this stage before it (exclusive,
-// counted from the start of [0, G), tile_off being the tile's offset) and
-// whether it is lost; the workgroup is the tile.  Every read of the tile
-// completes before the function returns (barriers of the scan).
-__device__ __forceinline__ void tile_prefix(const unsigned char* lpos, uint64_t G, unsigned char code,
-                                            uint64_t tile, uint64_t tile_off, uint64_t (&pre)[kPerThread],
-                                            bool (&bad)[kPerThread]) {
-    __shared__ unsigned s[kTileThreads];
-    const uint64_t base = tile * kTile + (uint64_t)threadIdx.x * kPerThread;
-    unsigned c = 0;
-    for (int k = 0; k < kPerThread; ++k) {
-        const uint64_t p = base + k;
-        bad[k] = p < G && lpos[p] == code;
-        c += bad[k] ? 1u : 0u;
+// bad: this thread's mask of lost rays of the stage in tile `tile`
+// (code_mask); returns the lost rays before its first position, counted from
+// the start of [0, G) (tile_off: the tile's offset).  The workgroup is the
+// tile; every read of the tile completes before the function returns
+// (barrier).
+__device__ __forceinline__ uint64_t tile_prefix(const unsigned char* lpos, uint64_t G, unsigned char code,
+                                                uint64_t tile, uint64_t tile_off, unsigned& bad) {
+    __shared__ unsigned s[kTileThreads / 64];
+    bad = code_mask(lpos, tile * kTile + (uint64_t)threadIdx.x * kPerThread, G, code);
+    const unsigned c = __popc(bad), lane = __lane_id();
+    unsigned run = c;                                    // inclusive scan over the wave
+    for (int off = 1; off < 64; off <<= 1) {
+        const unsigned t = __shfl_up(run, off);
+        if (lane >= (unsigned)off) run += t;
     }
-    s[threadIdx.x] = c;
+    if (lane == 63) s[threadIdx.x / 64] = run;
     __syncthreads();
-    for (int off = 1; off < kTileThreads; off <<= 1) {
-        const unsigned t = threadIdx.x >= (unsigned)off ? s[threadIdx.x - off] : 0u;
-        __syncthreads();
-        s[threadIdx.x] += t;
-        __syncthreads();
-    }
-    uint64_t run = tile_off + s[threadIdx.x] - c;
-    for (int k = 0; k < kPerThread; ++k) {
-        pre[k] = run;
-        run += bad[k] ? 1u : 0u;
-    }
+    for (unsigned w = 0; w < threadIdx.x / 64; ++w) run += s[w];
+    return tile_off + run - c;
 }
 
 // good rays of [G', G): the k-th from the back (k = 1, 2, ...) at gpos[k - 1];
@@ -146,16 +170,18 @@ __global__ __launch_bounds__(kTileThreads) void rt_stage_tail_kernel(const unsig
                                                                      const uint64_t* tile_off, uint64_t first_tile,
                                                                      uint64_t* gpos) {
     const uint64_t tile = first_tile + blockIdx.x;
-    uint64_t pre[kPerThread];
-    bool bad[kPerThread];
-    tile_prefix(lpos, G, code, tile, tile_off[tile], pre, bad);
+    unsigned bad;
+    uint64_t pre = tile_prefix(lpos, G, code, tile, tile_off[tile], bad);
     const uint64_t base = tile * kTile + (uint64_t)threadIdx.x * kPerThread;
     for (int k = 0; k < kPerThread; ++k) {
         const uint64_t q = base + k;
-        if (q < Gn || q >= G || bad[k]) continue;
-        // lost rays after q: all of them but the pre[k] before q (q is good)
-        const uint64_t bad_after = nb - pre[k];
-        const uint64_t good_after = (G - 1 - q) - bad_after;
+        if ((bad >> k) & 1u) {
+            ++pre;
+            continue;
+        }
+        if (q < Gn || q >= G) continue;
+        // lost rays after q: all of them but the `pre` before q (q is good)
+        const uint64_t good_after = (G - 1 - q) - (nb - pre);
         gpos[good_after] = q;
     }
 }
@@ -164,14 +190,13 @@ __global__ __launch_bounds__(kTileThreads) void rt_stage_tail_kernel(const unsig
 __global__ __launch_bounds__(kTileThreads) void rt_stage_head_kernel(unsigned char* lpos, uint64_t G, uint64_t Gn,
                                                                      unsigned char code, const uint64_t* tile_off,
                                                                      const uint64_t* gpos, uint64_t* perm) {
-    uint64_t pre[kPerThread];
-    bool bad[kPerThread];
-    tile_prefix(lpos, G, code, blockIdx.x, tile_off[blockIdx.x], pre, bad);
+    unsigned bad;
+    uint64_t pre = tile_prefix(lpos, G, code, blockIdx.x, tile_off[blockIdx.x], bad);
     const uint64_t base = (uint64_t)blockIdx.x * kTile + (uint64_t)threadIdx.x * kPerThread;
-    for (int k = 0; k < kPerThread; ++k) {
-        const uint64_t p = base + k;
-        if (p >= Gn || !bad[k]) continue;
-        const uint64_t q = gpos[pre[k]];
+    for (; bad; bad &= bad - 1) {
+        const uint64_t p = base + (uint64_t)(__ffs((int)bad) - 1);
+        if (p >= Gn) break;
+        const uint64_t q = gpos[pre++];
         const uint64_t rp = perm[p], rq = perm[q];
         perm[p] = rq;
         perm[q] = rp;
@@ -183,7 +208,7 @@ __global__ __launch_bounds__(kTileThreads) void rt_stage_head_kernel(unsigned ch
 
 // Beam::Normalize on one ray (beam.cpp:541-569): the scaled norm, in the
 // reference's operation order with no contraction
-__device__ __attribute__((noinline)) void normalize_reference(double& cX, double& cY, double& cZ) {
+__device__ __forceinline__ void normalize_reference(double& cX, double& cY, double& cZ) {
 #pragma clang fp contract(off)
     const double acX = fabs(cX), acY = fabs(cY), acZ = fabs(cZ);
     double norm;
@@ -208,14 +233,26 @@ struct OrderArgs {
     unsigned char renorm[256];
 };
 
+// Bound by the 7 rows read and written and the permutation (121 bytes a ray);
+// the rows' loads are issued together, the renormalisation counts read from
+// LDS (indexed in the argument segment they went through scratch memory, with
+// the rows behind a call: 82 us at 2e6 rays, now 56).
 __global__ __launch_bounds__(256) void rt_beam_order_kernel(OrderArgs a) {
+    __shared__ unsigned char s_renorm[256];
+    typedef const __attribute__((address_space(4))) unsigned char* cbytes;
+    if (threadIdx.x < 256)
+        s_renorm[threadIdx.x] = ((cbytes)__builtin_amdgcn_kernarg_segment_ptr())[__builtin_offsetof(OrderArgs, renorm) +
+                                                                                 threadIdx.x];
+    __syncthreads();
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; p < a.n; p += stride) {
         const uint64_t r = a.perm[p];
         double v[7];
+#pragma unroll
         for (int k = 0; k < 7; ++k) v[k] = a.in[k][r];
-        const int m = a.renorm[a.loss[r]];
+        const int m = s_renorm[a.loss[r]];
         for (int j = 0; j < m; ++j) normalize_reference(v[3], v[4], v[5]);
+#pragma unroll
         for (int k = 0; k < 7; ++k) a.out[(uint64_t)k * a.n + p] = v[k];
     }
 }
@@ -252,7 +289,7 @@ extern "C" int rt_hip_rearrange(const unsigned char* loss_dev, size_t n, uint64_
     WorkBufs& w = g_save_work.w;
     const uint64_t n_tiles = (n + kTile - 1) / kTile;
     if ((rc = w.ensure(WorkBufs::SAVE_HIST, 256 * sizeof(unsigned long long))) != RT_OK ||
-        (rc = w.ensure(WorkBufs::SAVE_LPOS, n)) != RT_OK ||
+        (rc = w.ensure(WorkBufs::SAVE_LPOS, n_tiles * kTile)) != RT_OK ||
         (rc = w.ensure(WorkBufs::SAVE_TILES, n_tiles * sizeof(uint64_t))) != RT_OK ||
         (rc = w.ensure(WorkBufs::SAVE_GPOS, n * sizeof(uint64_t))) != RT_OK)
         return rc;
@@ -263,9 +300,11 @@ extern "C" int rt_hip_rearrange(const unsigned char* loss_dev, size_t n, uint64_
     uint64_t* gpos = w.get<uint64_t>(WorkBufs::SAVE_GPOS);
 
     hipLaunchKernelGGL(rt_save_zero_kernel, dim3(1), dim3(256), 0, st, hist, 256);
-    hipLaunchKernelGGL(rt_loss_hist_kernel, dim3(grid_for(n, 256)), dim3(256), 0, st, loss_dev, (uint64_t)n, hist);
-    hipLaunchKernelGGL(rt_order_init_kernel, dim3(grid_for(n, 256)), dim3(256), 0, st, loss_dev, (uint64_t)n,
-                       perm_dev, lpos);
+    const int V = ((uintptr_t)loss_dev & 3u) == 0 ? 4 : 1;
+    const uint64_t want = (n + (uint64_t)kInitThreads * V - 1) / ((uint64_t)kInitThreads * V);
+    hipLaunchKernelGGL(V == 4 ? rt_order_init_kernel<4> : rt_order_init_kernel<1>,
+                       dim3((unsigned)std::min<uint64_t>(want, kInitBlocks)), dim3(kInitThreads), 0, st, loss_dev,
+                       (uint64_t)n, perm_dev, lpos, hist);
     if (hipGetLastError() != hipSuccess) return rt_set_error(RT_ERR_FAILED, "rearrange launch failed");
     if (hipMemcpyAsync(counts, hist, 256 * sizeof(uint64_t), hipMemcpyDeviceToHost, st) != hipSuccess ||
         hipStreamSynchronize(st) != hipSuccess)

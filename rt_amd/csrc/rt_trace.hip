@@ -107,17 +107,27 @@ __global__ __launch_bounds__(kBlock) void rt_trace_kernel(TraceArgs a) {
     });
 }
 
-// extents keys before a recording trace: min keys all ones, max keys zero
-__global__ void rt_ext_init_kernel(unsigned long long* keys, int n) {
-    for (int i = threadIdx.x; i < n; i += blockDim.x) keys[i] = (i & 1) ? 0ull : ~0ull;
-}
-
-// extents as doubles (NaN where no ray was alive)
-__global__ void rt_ext_decode_kernel(const unsigned long long* keys, int n, double* out) {
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        const unsigned long long k = keys[i];
-        const bool empty = (i & 1) ? k == 0ull : k == ~0ull;
-        out[i] = empty ? __builtin_nan("") : rt::key_value(k);
+// Extents of a recording trace from its workgroups' keys (key k of workgroup w
+// at keys[k * n_wg + w]; even k a minimum, odd k the minimum of the negated
+// value, see rt::ext_add), as doubles, NaN where no ray was alive; workgroup
+// blockIdx.x = key k.
+__global__ __launch_bounds__(256) void rt_ext_reduce_kernel(const unsigned long long* keys, unsigned n_wg,
+                                                            double* out) {
+    __shared__ unsigned long long s[256];
+    unsigned long long v = ~0ull;
+    for (unsigned w = threadIdx.x; w < n_wg; w += 256) {
+        const unsigned long long k = keys[(size_t)blockIdx.x * n_wg + w];
+        v = k < v ? k : v;
+    }
+    s[threadIdx.x] = v;
+    __syncthreads();
+    for (int m = 128; m > 0; m >>= 1) {
+        if ((int)threadIdx.x < m && s[threadIdx.x + m] < s[threadIdx.x]) s[threadIdx.x] = s[threadIdx.x + m];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        const double d = rt::key_value(s[0]);
+        out[blockIdx.x] = s[0] == ~0ull ? __builtin_nan("") : (blockIdx.x & 1) ? -d : d;
     }
 }
 
@@ -942,12 +952,20 @@ static void beam_uniforms(TraceArgs& a) {
 }
 
 namespace {
+// The workgroups of a recording trace with extents: as many as are resident
+// at once and no more, so that each walks many rays under bounds it has met
+// (ext_add) and leaves one row of keys, in whole rounds of rays.
+unsigned ext_grid(uint64_t tiles, uint64_t resident) {
+    const uint64_t rounds = (tiles + resident - 1) / resident;
+    return (unsigned)((tiles + rounds - 1) / rounds);
+}
+
 // rt_hip_trace and rt_hip_trace_record: rec is the recording mode (rt::kRecLoss
-// | rt::kRecExt or 0), loss / ext_keys its outputs
+// | rt::kRecExt or 0), loss / extents its outputs
 int trace_launch(const rt_hip_scheme* sch, const double* beam_desc, uint64_t seed, size_t ray_begin, size_t n_rays,
                  double* X, double* Y, double* Z, double* cX, double* cY, double* cZ, double* lambda,
                  signed char* flag, int flags, unsigned int* ccd_hist, double* ccd_flux, unsigned long long* stats,
-                 double* dump, signed char* dump_flag, int rec, unsigned char* loss, unsigned long long* ext_keys,
+                 double* dump, signed char* dump_flag, int rec, unsigned char* loss, double* extents,
                  void* stream, double* group_part = nullptr, uint64_t n_groups = 0, int* block_used = nullptr) {
     if (!sch) return set_error(RT_ERR_BAD_VALUE, "scheme is NULL");
     const bool gen = (flags & RT_TRACE_GENERATE) != 0;
@@ -983,7 +1001,6 @@ int trace_launch(const rt_hip_scheme* sch, const double* beam_desc, uint64_t see
     a.hist = ccd_hist; a.flux = ccd_flux; a.dump = dump; a.dump_flag = dump_flag;
     a.stats = stats ? sch->stat_copies : nullptr;
     a.loss = loss;
-    a.ext = ext_keys;
     a.group_part = group_part;
     a.n_groups = n_groups;
 
@@ -993,6 +1010,14 @@ int trace_launch(const rt_hip_scheme* sch, const double* beam_desc, uint64_t see
     const int beam_mode = gen ? (int)a.beam.v[RT_B_TYPE] : kLoad;
 
     const uint64_t nk = gen && sch->unroll ? dtab_nk(sch->dt, beam_desc) : 0;
+    unsigned grid = 0;
+    // the rows of extents keys of as many workgroups as this launch can have
+    auto ext_rows = [&](uint64_t most) {
+        const int r = sch->work.ensure(WorkBufs::EXT_KEYS,
+                                       (size_t)sch->n_surf * rt::kExtPerSurf * most * sizeof(unsigned long long));
+        if (r == RT_OK) a.ext = sch->work.get<unsigned long long>(WorkBufs::EXT_KEYS);
+        return r;
+    };
     hipFunction_t fn = nullptr;
     if (rt_jit_enabled() && sch->unroll)
         fn = rt_jit_kernel(sch->signature, beam_mode | (nk ? RT_JIT_LTAB : 0),
@@ -1015,7 +1040,12 @@ int trace_launch(const rt_hip_scheme* sch, const double* beam_desc, uint64_t see
             resident = 1;
         uint64_t want = (n_rays + sch->block - 1) / sch->block;
         uint64_t cap = (uint64_t)cus * resident * sch->grid_mult;
-        unsigned grid = (unsigned)(want < cap ? want : cap);
+        grid = (unsigned)(want < cap ? want : cap);
+        if (extents) {
+            grid = ext_grid(want, (uint64_t)cus * resident);
+            rc = ext_rows((uint64_t)cus * resident);
+            if (rc != RT_OK) return rc;
+        }
         void* params[] = {&a};
         HIP_TRY(hipModuleLaunchKernel(fn, grid, 1, 1, sch->block, 1, 1, (unsigned)lds, st, params, nullptr),
                 RT_ERR_FAILED);
@@ -1028,7 +1058,12 @@ int trace_launch(const rt_hip_scheme* sch, const double* beam_desc, uint64_t see
     } else {
         uint64_t want = (n_rays + kBlock - 1) / kBlock;
         uint64_t cap = (uint64_t)cus * 8;      // persistent grid: 8 blocks (32 waves) per CU
-        unsigned grid = (unsigned)(want < cap ? want : cap);
+        grid = (unsigned)(want < cap ? want : cap);
+        if (extents) {
+            grid = ext_grid(want, cap);
+            rc = ext_rows(cap);
+            if (rc != RT_OK) return rc;
+        }
         constexpr int R = rt::kRecLoss | rt::kRecExt, SP = rt::kRecSpots;
         auto kern = rec == 0 ? (beam_mode == RT_BEAM_PARALLEL ? rt_trace_kernel<RT_BEAM_PARALLEL>
                                 : beam_mode == RT_BEAM_CONIC  ? rt_trace_kernel<RT_BEAM_CONIC>
@@ -1048,6 +1083,11 @@ int trace_launch(const rt_hip_scheme* sch, const double* beam_desc, uint64_t see
             fprintf(stderr, "rt_hip: trace generic kernel, %zu rays, grid %u, record %d\n", n_rays, grid, rec);
     }
     HIP_TRY(hipGetLastError(), RT_ERR_FAILED);
+    if (extents) {
+        hipLaunchKernelGGL(rt_ext_reduce_kernel, dim3((unsigned)(sch->n_surf * rt::kExtPerSurf)), dim3(256), 0, st,
+                           (const unsigned long long*)a.ext, grid, extents);
+        HIP_TRY(hipGetLastError(), RT_ERR_FAILED);
+    }
     if (stats) return stats_fold(sch->stat_copies, stats, st);
     return RT_OK;
 }
@@ -1106,24 +1146,11 @@ extern "C" int rt_hip_trace_record(const rt_hip_scheme* sch, const double* beam_
     int rc = ensure_device();
     if (rc != RT_OK) return rc;
     hipStream_t st = (hipStream_t)stream;
-    const int n_ext = sch->n_surf * rt::kExtPerSurf;
-    unsigned long long* keys = nullptr;
-    if (extents) {
-        rc = sch->work.ensure(WorkBufs::EXT_KEYS, (size_t)rt::kExtPerSurf * RT_MAX_SURF * sizeof(unsigned long long));
-        if (rc != RT_OK) return rc;
-        keys = sch->work.get<unsigned long long>(WorkBufs::EXT_KEYS);
-        hipLaunchKernelGGL(rt_ext_init_kernel, dim3(1), dim3(256), 0, st, keys, n_ext);
-        HIP_TRY(hipGetLastError(), RT_ERR_FAILED);
-    }
     rc = trace_launch(sch, beam_desc, seed, 0, n_rays, X, Y, Z, cX, cY, cZ, lambda, flag, flags, nullptr, nullptr,
-                      stats, nullptr, nullptr, rt::kRecLoss | (extents ? rt::kRecExt : 0), loss, keys, stream);
-    if (rc != RT_OK || !extents) return rc;
-    if (n_rays == 0) {
-        hipLaunchKernelGGL(rt_ext_init_kernel, dim3(1), dim3(256), 0, st, keys, n_ext);
-        HIP_TRY(hipGetLastError(), RT_ERR_FAILED);
-    }
-    hipLaunchKernelGGL(rt_ext_decode_kernel, dim3(1), dim3(256), 0, st, (const unsigned long long*)keys, n_ext,
-                       extents);
+                      stats, nullptr, nullptr, rt::kRecLoss | (extents ? rt::kRecExt : 0), loss, extents, stream);
+    if (rc != RT_OK || !extents || n_rays > 0) return rc;
+    hipLaunchKernelGGL(rt_ext_reduce_kernel, dim3((unsigned)(sch->n_surf * rt::kExtPerSurf)), dim3(256), 0, st,
+                       (const unsigned long long*)nullptr, 0u, extents);           // no ray: every extent empty
     HIP_TRY(hipGetLastError(), RT_ERR_FAILED);
     return RT_OK;
 }

@@ -99,3 +99,66 @@ def test_transform_touches_what_it_moves(hip, dist, ang):
         else:
             # up to three rotations of values near 150: a few units of 150 * 2^-53
             assert np.allclose(got[k], want[k], rtol=0.0, atol=3e-13, equal_nan=True), k
+
+
+def reference_order(codes):
+    """Beam::Rearrange after every stage that lost rays, one swap at a time"""
+    perm, G = list(range(len(codes))), len(codes)
+    for c in range(1, 255):
+        bad = [codes[r] == c for r in perm[:G]]
+        if not any(bad):
+            continue
+        i, j = 0, G - 1
+        while True:
+            while i < G and not bad[i]:
+                i += 1
+            while j >= 0 and bad[j]:
+                j -= 1
+            if i >= j:
+                break
+            perm[i], perm[j] = perm[j], perm[i]
+            bad[i], bad[j] = bad[j], bad[i]
+        G -= sum(bad)
+    return perm
+
+
+# a tile is 4096 positions of 16 a lane; codes read four at a time from an
+# aligned start, one at a time from any other
+@pytest.mark.parametrize("n,offset", [(1, 0), (3, 0), (17, 1), (4095, 0), (4096, 0), (4097, 2), (3 * 4096 + 7, 3)])
+@pytest.mark.parametrize("lost", [0.01, 0.6, 1.0])
+def test_rearrange_order_and_counts(hip, n, offset, lost):
+    print(f"[rearrange] n={n} offset={offset} lost={lost}", flush=True)
+    rng = np.random.default_rng(n)
+    codes = np.where(rng.random(n) < lost, rng.integers(1, 9, n), 0).astype(np.uint8)
+    dev = torch.zeros(n + offset, dtype=torch.uint8, device="cuda")
+    dev[offset:].copy_(torch.from_numpy(codes))
+    perm, counts = hip.rearrange(dev[offset:])
+    assert np.array_equal(perm.cpu().numpy(), reference_order(codes))
+    assert np.array_equal(counts, np.bincount(codes, minlength=256))
+
+
+# one ray, a partial workgroup, and more rays than the resident workgroups take
+# in one round (so that each meets rays inside and outside its bounds)
+@pytest.mark.parametrize("n", [1, 300, 700003])
+def test_recorded_extents_equal_dumped_states(hip, n):
+    print(f"[extents] n={n}", flush=True)
+    from rt_amd import scheme as S, schemes
+    sc = schemes.echelle_fixed_order(n, 1)
+    ds = hip.DeviceScheme(sc)
+    rays, flag = torch.empty((7, n), dtype=torch.float64, device="cuda"), torch.empty(n, dtype=torch.int8, device="cuda")
+    loss = torch.empty(n, dtype=torch.uint8, device="cuda")
+    ext = torch.zeros((sc.n_surf, hip.EXT_PER_SURF), dtype=torch.float64, device="cuda")
+    ds.trace_record(rays, flag, loss, seed=4, extents=ext)
+    dump = torch.empty((sc.n_surf, 7, n), dtype=torch.float64, device="cuda")
+    dflag = torch.empty((sc.n_surf, n), dtype=torch.int8, device="cuda")
+    ds.trace(None, None, seed=4, n=n, flags=S.RT_TRACE_GENERATE, dump=dump, dump_flag=dflag)
+    e, codes = ext.cpu().numpy(), loss.cpu().numpy()
+    for s in range(sc.n_surf):
+        st, alive = dump[s].cpu().numpy(), dflag[s].cpu().numpy() != 0
+        # X, Y after the aperture: the rays past it, those lost at the action too
+        passed = alive | (codes == 3 + 3 * s)
+        for q, row, on in ((3, 0, passed), (4, 1, passed), (5, 5, alive)):
+            v = st[row][on]
+            want = (v.min(), v.max()) if v.size else (np.nan, np.nan)
+            assert np.array_equal(e[s, 2 * q:2 * q + 2], want, equal_nan=True), (s, q)
+    ds.close()
