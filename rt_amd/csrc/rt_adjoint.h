@@ -81,7 +81,7 @@ RT_HD double dinvnorm(double s) {
 #if defined(__HIP_DEVICE_COMPILE__)
     const double d = s - 1.0;
     const bool near = fabs(d) < 1e-8;
-    if (__all(near)) return fma(-0.5, d, 1.0);
+    if (rt::wave_all(near)) return fma(-0.5, d, 1.0);
     return near ? fma(-0.5, d, 1.0) : rt::rsqrt(s);
 #else
     return 1.0 / sqrt(s);
@@ -1079,7 +1079,7 @@ __device__ __forceinline__ void adjoint_body(const AdjArgs& a, Fwd forward, Bwd 
     c.hist = nullptr;
     c.flux = nullptr;
     c.do_hist = c.do_flux = false;
-    c.n_oob = c.n_hit = c.n_off = c.n_edge = 0;
+    c.n_rays = c.n_dead = c.n_oob = c.n_off = c.n_edge = 0;
     c.n_prev = 0.0;
     c.last_it = 0;
     const uint64_t G = (uint64_t)gridDim.x * blockDim.x;      // lanes (blockDim a multiple of 64)
@@ -1102,13 +1102,9 @@ __device__ __forceinline__ void adjoint_body(const AdjArgs& a, Fwd forward, Bwd 
         gen_ray<BEAM>(bm, a.seed, i, r, jl);
         c.lk = (uint32_t)jl;
         bool alive = in;
+        c.n_rays += in ? 1u : 0u;
         forward(r, alive, c, lane_rows(a.tape, a.tape_rows, G, lane));
-        unsigned long long good = __ballot(alive), all = __ballot(in);
-        if (lw == 0) {
-            atomicAdd(&s_stats[RT_ST_RAYS], (unsigned)__popcll(all));
-            if (good) atomicAdd(&s_stats[RT_ST_GOOD], (unsigned)__popcll(good));
-        }
-        if (!good) continue;                                   // wave-uniform
+        if (!wave_ballot(alive)) continue;                        // wave-uniform
         const uint64_t g = i % a.n_groups;
         const double bx = a.seeds[3 * g], by = a.seeds[3 * g + 1], b = a.seeds[3 * g + 2];
         St ad = {bx + b * r.X, by + b * r.Y, 0.0, 0.0, 0.0, 0.0};
@@ -1116,12 +1112,9 @@ __device__ __forceinline__ void adjoint_body(const AdjArgs& a, Fwd forward, Bwd 
         if (alive && !ok) ++skipped;
     }
     acc.end(a, wave, W, lw);
-    lds_add(&s_stats[RT_ST_SPLINE_OOB], c.n_oob);
-    lds_add(&s_stats[RT_ST_ADJ_SKIP], skipped);
-    __syncthreads();
     if (a.stats) {
-        for (int k = threadIdx.x; k < RT_STATS_LEN; k += blockDim.x)
-            if (s_stats[k]) atomicAdd(&a.stats[k], (unsigned long long)s_stats[k]);
+        lds_add(&s_stats[RT_ST_ADJ_SKIP], skipped);
+        flush_counts(c, a.stats, true, a.table, a.n_surf);
     }
 }
 
@@ -1144,7 +1137,7 @@ __device__ __forceinline__ void adjoint_batch_body(const AdjArgs& a, Fwd forward
     c.hist = nullptr;
     c.flux = nullptr;
     c.do_hist = c.do_flux = false;
-    c.n_oob = c.n_hit = c.n_off = c.n_edge = 0;
+    c.n_rays = c.n_dead = c.n_oob = c.n_off = c.n_edge = 0;
     c.n_prev = 0.0;
     c.last_it = 0;
     const uint64_t G = (uint64_t)gridDim.x * blockDim.x;      // tape lanes
@@ -1181,12 +1174,8 @@ __device__ __forceinline__ void adjoint_batch_body(const AdjArgs& a, Fwd forward
         gen_ray<BEAM>(bm, ka->seed + inst, r, ray, jl);
         c.lk = (uint32_t)jl;
         bool alive = in;
+        c.n_rays += in ? 1u : 0u;
         forward(ray, alive, c, lane_rows(a.tape, a.tape_rows, G, lane));
-        unsigned long long good = __ballot(alive), all = __ballot(in);
-        if (lw == 0) {
-            if (all) atomicAdd(&s_stats[RT_ST_RAYS], (unsigned)__popcll(all));
-            if (good) atomicAdd(&s_stats[RT_ST_GOOD], (unsigned)__popcll(good));
-        }
         const uint64_t g = r % ka->n_groups;
         const double* sd = ka->seeds + (inst * ka->n_groups + g) * 3;
         const double bx = sd[0], by = sd[1], b = sd[2];
@@ -1196,12 +1185,9 @@ __device__ __forceinline__ void adjoint_batch_body(const AdjArgs& a, Fwd forward
         if (alive && !ok) ++skipped;
         acc.tile_end(a, t * wpg + wib, lw);
     }
-    lds_add(&s_stats[RT_ST_SPLINE_OOB], c.n_oob);
-    lds_add(&s_stats[RT_ST_ADJ_SKIP], skipped);
-    __syncthreads();
     if (a.stats) {
-        for (int k = threadIdx.x; k < RT_STATS_LEN; k += blockDim.x)
-            if (s_stats[k]) atomicAdd(&a.stats[k], (unsigned long long)s_stats[k]);
+        lds_add(&s_stats[RT_ST_ADJ_SKIP], skipped);
+        flush_counts(c, a.stats, true, a.table, a.n_surf);
     }
 }
 

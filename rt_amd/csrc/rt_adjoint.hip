@@ -333,7 +333,9 @@ extern "C" int rt_hip_adjoint(const rt_hip_scheme* sch, const double* beam_desc,
     auto kern = beam_type == RT_BEAM_PARALLEL ? rt_adjoint_kernel<RT_BEAM_PARALLEL>
               : beam_type == RT_BEAM_CONIC    ? rt_adjoint_kernel<RT_BEAM_CONIC>
                                               : rt_adjoint_kernel<RT_BEAM_GAUSS>;
-    const size_t lds = pool_len * sizeof(double);
+    // the table's kernels read no spline
+    const size_t lds = fn && nk ? 0 : pool_len * sizeof(double);
+    if (fn && nk) a.pool_len = 0;
     int resident = 0;
     hipError_t oe = fn ? hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&resident, fn, kAdjBlock, lds)
                        : hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, kern, kAdjBlock, lds);
@@ -440,7 +442,9 @@ extern "C" int rt_hip_batch_adjoint(const rt_hip_batch* b, const double* beam_de
     auto kern = beam_type == RT_BEAM_PARALLEL ? rt_adjoint_batch_kernel<RT_BEAM_PARALLEL>
               : beam_type == RT_BEAM_CONIC    ? rt_adjoint_batch_kernel<RT_BEAM_CONIC>
                                               : rt_adjoint_batch_kernel<RT_BEAM_GAUSS>;
-    const size_t lds = v.pool_len * sizeof(double);
+    // the table's kernels read no spline
+    const size_t lds = fn && nk ? 0 : v.pool_len * sizeof(double);
+    if (fn && nk) a.pool_len = 0;
     int resident = 0;
     hipError_t oe = fn ? hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&resident, fn, kAdjBlock, lds)
                        : hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, kern, kAdjBlock, lds);

@@ -31,6 +31,12 @@ struct Ray {
     double X, Y, Z, cX, cY, cZ, lam;
 };
 
+// The lanes of the wave that are here and for which p holds, and whether it
+// holds for all of them: the compare's own lane mask (the run-time compiler
+// makes a select and a second compare of HIP's ballot and all votes).
+__device__ __forceinline__ uint64_t wave_ballot(bool p) { return __builtin_amdgcn_ballot_w64(p); }
+__device__ __forceinline__ bool wave_all(bool p) { return __builtin_amdgcn_ballot_w64(!p) == 0; }
+
 // Read-only kernel data (surface records, beam description) is read through
 // the constant address space, so wave-uniform reads become scalar loads.
 typedef const __attribute__((address_space(4))) double* cptr;
@@ -115,10 +121,15 @@ struct StatSurf {
 };
 
 // ------------------------------------------------------------- FP64 math
-// The hardware reciprocal / reciprocal square root estimates refined by two
-// Newton-Raphson steps each (quadratic convergence: any estimate better than
-// 2^-14 reaches the FP64 rounding floor), about 1 ulp from the IEEE result
-// at a third of the instructions of the IEEE division sequence.
+// The hardware estimates v_rcp_f64 and v_rsq_f64 (relative error below 5.3e-8
+// over 2.7e8 random arguments) refined to the FP64 rounding floor: one step of
+// third order, 1 + e + e^2 for the reciprocal and 1 + e/2 + 3e^2/8 for the
+// reciprocal square root, leaves e^3 < 2^-72 of the error.  Against two
+// Newton-Raphson steps that is one instruction less per reciprocal and two
+// less per reciprocal square root, with the same largest errors over those
+// arguments (1.00 and 1.25 x 2^-53; quotient and square root equal the IEEE
+// results on all of them, before and after).  The traces are bound by VALU
+// issue and take about 75 of these per ray.
 // Reciprocals and quotients take their special values from v_div_fixup_f64,
 // the instruction that ends the IEEE division sequence: for a zero, infinite
 // or NaN operand it returns the IEEE quotient (x/0 = inf, x/inf = 0, 0/0 and
@@ -132,64 +143,62 @@ __device__ __forceinline__ bool finite_nonzero(double r) {
 
 // 1/x refined, for x finite and away from zero (a zero or infinite x gives NaN)
 __device__ __forceinline__ double rcp_fin(double x) {
-    double r = __builtin_amdgcn_rcp(x);
-    double e = fma(-x, r, 1.0);
-    double q = fma(r, e, r);
-    e = fma(-x, q, 1.0);
-    return fma(q, e, q);
+    const double r = __builtin_amdgcn_rcp(x);
+    const double e = fma(-x, r, 1.0);
+    return fma(r, fma(e, e, e), r);
 }
 
 __device__ __forceinline__ double rcp(double x) {
     return __builtin_amdgcn_div_fixup(rcp_fin(x), x, 1.0);
 }
 
-// a / b: the refined reciprocal, the product and one residual correction
+// a / b: a reciprocal good to 2^-48, the product and one residual correction
+// (which squares that error)
 __device__ __forceinline__ double fdiv(double a, double b) {
-    const double r = rcp_fin(b);
+    double r = __builtin_amdgcn_rcp(b);
+    r = fma(r, fma(-b, r, 1.0), r);
     const double q = a * r;
     return __builtin_amdgcn_div_fixup(fma(fma(-b, q, a), r, q), b, a);
 }
 
+// 1/sqrt(x) for x > 0 finite; x <= 0, infinite or NaN gives NaN (the Newton
+// loops end on it)
+__device__ __forceinline__ double rsqrt_pos(double x) {
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-(x * y), y, 1.0);
+    return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+
+// 1/sqrt(x) with the IEEE values at 0 and infinity
 __device__ __forceinline__ double rsqrt(double x) {
-    double y = __builtin_amdgcn_rsq(x);
-    double h = 0.5 * x;
-    double e = fma(-h * y, y, 0.5);
-    double z = fma(y, e, y);
-    e = fma(-h * z, z, 0.5);
-    z = fma(z, e, z);
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-(x * y), y, 1.0);
+    const double z = fma(y * e, fma(e, 0.375, 0.5), y);
     return finite_nonzero(y) ? z : y;
 }
 
-// sqrt(x) from x * rsqrt(x) with one residual correction; x = +-0 and +inf
-// return x (the IEEE results), negative and NaN x give NaN through ry
-__device__ __forceinline__ double fsqrt_with(double x, double ry) {
-    double s = x * ry;
-    double t = fma(-s, s, x);
-    s = fma(t, 0.5 * ry, s);
+// sqrt(x), x > 0 finite, from ry = rsqrt_pos(x): x ry with one residual correction
+__device__ __forceinline__ double fsqrt_pos(double x, double ry) {
+    const double s = x * ry;
+    return fma(fma(-s, s, x), 0.5 * ry, s);
+}
+
+// sqrt(x): s -> sqrt(x) and h -> 1/(2 sqrt(x)) refined together (Goldschmidt)
+// to 2^-47, then one residual correction of s, which squares that; x = +-0 and
+// +inf return x (the IEEE results), negative and NaN x give NaN
+__device__ __forceinline__ double fsqrt(double x) {
+    const double y = __builtin_amdgcn_rsq(x);
+    double s = x * y, h = 0.5 * y;
+    const double e = fma(-h, s, 0.5);
+    s = fma(s, e, s);
+    h = fma(h, e, h);
+    s = fma(fma(-s, s, x), h, s);
     constexpr int kZeroOrPosInf = (1 << 5) | (1 << 6) | (1 << 9);    // v_cmp_class: -0, +0, +inf
     return __builtin_amdgcn_class(x, kZeroOrPosInf) ? x : s;
 }
 
-__device__ __forceinline__ double fsqrt(double x) { return fsqrt_with(x, rsqrt(x)); }
-
 // a / b for b finite, nonzero (the same sequence as fdiv)
 __device__ __forceinline__ double fdiv_fin(double a, double b) { return fdiv(a, b); }
-
-// 1/sqrt(x) for x > 0 finite; x <= 0 gives NaN (the Newton loops end on it)
-__device__ __forceinline__ double rsqrt_pos(double x) {
-    double y = __builtin_amdgcn_rsq(x);
-    double h = 0.5 * x;
-    double e = fma(-h * y, y, 0.5);
-    double z = fma(y, e, y);
-    e = fma(-h * z, z, 0.5);
-    return fma(z, e, z);
-}
-
-__device__ __forceinline__ double fsqrt_pos(double x, double ry) {
-    double s = x * ry;
-    double t = fma(-s, s, x);
-    return fma(t, 0.5 * ry, s);
-}
 
 // sin and cos of an angle of moderate size (|x| < 2^20; the beam generators
 // use |x| <= 2 pi): Cody-Waite reduction to r = x - k pi/2, |r| <= pi/4, with
@@ -289,10 +298,10 @@ __device__ __forceinline__ void philox4x32_10(uint32_t c0, uint32_t c1, uint32_t
     out[0] = c0; out[1] = c1; out[2] = c2; out[3] = c3;
 }
 
-// (0,1] from 64 random bits: (top 53 bits + 1) * 2^-53
+// (0,1] from 64 random bits: (top 53 bits + 1) * 2^-53, as hi 2^-32 + (lo /
+// 2^11 + 1) 2^-53: both terms exact, and their sum has at most 53 bits
 __device__ __forceinline__ double u01(uint32_t hi, uint32_t lo) {
-    uint64_t v = ((((uint64_t)hi) << 32) | lo) >> 11;
-    return (double)(v + 1) * (1.0 / 9007199254740992.0);
+    return fma((double)hi, 0x1p-32, (double)((lo >> 11) + 1u) * 0x1p-53);
 }
 
 __device__ __forceinline__ void philox_stream(uint64_t seed, uint64_t idx, uint32_t stream,
@@ -551,9 +560,8 @@ __device__ __forceinline__ void normalize_ray(double& cX, double& cY, double& cZ
     const double s = cX * cX + cY * cY + cZ * cZ;
     const double d = s - 1.0;
     const bool near = fabs(d) < 1e-8;
-    double inv;
-    if (__all(near)) inv = fma(-0.5, d, 1.0);
-    else inv = near ? fma(-0.5, d, 1.0) : rsqrt(s);
+    double inv = fma(-0.5, d, 1.0);
+    if (!wave_all(near)) inv = near ? inv : rsqrt(s);
     cX *= inv; cY *= inv; cZ *= inv;
 }
 
@@ -575,37 +583,73 @@ __device__ __forceinline__ void asphere_pq(const SD& d, double r2, double& P, do
     Q = qa;
 }
 
-// conic_derivs (surface.cu:45-61)
+// The surface's profile where an iterating intersection met it: what its last
+// iteration evaluated at the point it returns, kept for the normal of the
+// action that follows (about 20 instructions a surface).  Conic: e the factor
+// of the normal, -dF/dX = e X; toric: f the profile F(Y), e its derivative.
+// The expressions are those of conic_derivs and toric_derivs, so the normal is
+// the same bit for bit.
+struct Profile {
+    double e = 0.0, f = 0.0;
+};
+
 template <class SD>
-__device__ __forceinline__ void conic_derivs(const SD& d, double X, double Y, double& dFdX, double& dFdY) {
-    const cptr p = d.p;
-    const double c = p[RT_S_C];
-    double r2 = X * X + Y * Y;
-    double E = c * rsqrt(1.0 - p[D_K1C2] * r2);
-    double P, Q;
-    asphere_pq(d, r2, P, Q);
-    E += 2.0 * Q;
+__device__ __forceinline__ bool has_profile(const SD& d) {
+    return d.ikind() == IK_CONIC_NEWTON || d.ikind() == IK_TORIC_NEWTON;
+}
+
+// the factor E = c / sqrt(1 - (k+1) c^2 r2) + 2 Q of the conic normal, from
+// irt = 1/sqrt(...) and the polynomial's derivative
+template <class SD>
+__device__ __forceinline__ double conic_factor(const SD& d, double irt, double Q) {
+    const double c = d.p[RT_S_C];
+    return d.npoly() == 0 ? c * irt : c * irt + 2.0 * Q;
+}
+
+// conic_derivs (surface.cu:45-61); given: the profile at the point, or null
+template <class SD>
+__device__ __forceinline__ void conic_derivs(const SD& d, double X, double Y, double& dFdX, double& dFdY,
+                                             const Profile* given = nullptr) {
+    double E;
+    if (given) {
+        E = given->e;
+    } else {
+        const double r2 = X * X + Y * Y;
+        const double irt = rsqrt_pos(1.0 - d.p[D_K1C2] * r2);
+        double P, Q;
+        asphere_pq(d, r2, P, Q);
+        E = conic_factor(d, irt, Q);
+    }
     dFdX = -E * X;
     dFdY = -E * Y;
 }
 
-// toric_derivs (surface.cu:65-94), asphere derivative with its factor Y (D18)
+// the toric's profile Fy at Y and its derivative with the asphere's factor Y
+// (D18), from t = 1 - (k+1) c^2 Y^2 and irt = 1/sqrt(t)
 template <class SD>
-__device__ __forceinline__ void toric_derivs(const SD& d, double X, double Y, double Z,
-                                             double& dFdX, double& dFdY, double& dFdZ) {
-    const cptr p = d.p;
-    const double c = p[RT_S_C], cR = p[RT_S_CR];
-    double Y2 = Y * Y;
-    double t = 1.0 - p[D_K1C2] * Y2;
-    double irt = rsqrt(t);
-    double Fy = fdiv(c * Y2, 1.0 + fsqrt_with(t, irt));
+__device__ __forceinline__ void toric_profile(const SD& d, double Y, double Y2, double t, double irt, Profile& o) {
+    const double c = d.p[RT_S_C];
     double P, Q;
     asphere_pq(d, Y2, P, Q);
-    Fy += P;
-    double dFy = c * Y * irt;
-    dFy += 2.0 * Q * Y;
+    const double w = rcp_fin(1.0 + fsqrt_pos(t, irt));
+    o.f = d.npoly() == 0 ? (c * Y2) * w : (c * Y2) * w + P;
+    o.e = d.npoly() == 0 ? c * Y * irt : c * Y * irt + 2.0 * Q * Y;
+}
+
+// toric_derivs (surface.cu:65-94); given: the profile at the point, or null
+template <class SD>
+__device__ __forceinline__ void toric_derivs(const SD& d, double X, double Y, double Z,
+                                             double& dFdX, double& dFdY, double& dFdZ, const Profile* given = nullptr) {
+    const double cR = d.p[RT_S_CR];
+    Profile o;
+    if (given) {
+        o = *given;
+    } else {
+        const double Y2 = Y * Y, t = 1.0 - d.p[D_K1C2] * Y2;
+        toric_profile(d, Y, Y2, t, rsqrt_pos(t), o);
+    }
     dFdX = -cR * X;
-    dFdY = (cR * Fy - 1.0) * dFy;
+    dFdY = (cR * o.f - 1.0) * o.e;
     dFdZ = 1.0 - cR * Z;
 }
 
@@ -620,8 +664,10 @@ struct NoIterSink {
 // surface.cu:593-636).  Returns false for a lost ray; `iters` counts Newton
 // iterations.  A lost Newton ray keeps its last iterate, as the reference
 // writes Xi,Yi,Zi before flagging (surface.cu:319-326).
+// prof: the profile at the point of an iterating intersection.
 template <class SD, class Sink = NoIterSink>
-__device__ __forceinline__ bool intersect_ray(const SD& d, Ray& r, unsigned& iters, const Sink& sink = Sink{}) {
+__device__ __forceinline__ bool intersect_ray(const SD& d, Ray& r, unsigned& iters, Profile& prof,
+                                              const Sink& sink = Sink{}) {
     const cptr p = d.p;
     const int ik = d.ikind();
     const double c = p[RT_S_C];
@@ -630,6 +676,7 @@ __device__ __forceinline__ bool intersect_ray(const SD& d, Ray& r, unsigned& ite
         // plane_intersection (surface.cu:154-178)
         double s0 = fdiv(-r.Z, r.cZ);
         if (s0 < 0.0) return false;
+        __asm__ volatile("");                    // a branch: not three selects of 64-bit values
         r.X += r.cX * s0;
         r.Y += r.cY * s0;
         r.Z = 0.0;
@@ -637,19 +684,22 @@ __device__ __forceinline__ bool intersect_ray(const SD& d, Ray& r, unsigned& ite
     }
     if (ik == IK_QUAD) {
         // conic_intersection (surface.cu:216-253), stable root (D7), root by sign(c) (D8)
+        // with B/2 in place of B: s = q/A or C/q, q = -(B/2 + sign(B) sqrt(B^2/4 - A C))
+        // (a scaling by powers of two: the same roots bit for bit)
         const double k1 = p[RT_S_K] + 1;
-        double A = k1 * r.cZ * r.cZ + r.cX * r.cX + r.cY * r.cY;
+        const double A = k1 * r.cZ * r.cZ + r.cX * r.cX + r.cY * r.cY;
         const double ic = p[D_INV_C];
-        double B = 2.0 * (k1 * r.Z * r.cZ + r.X * r.cX + r.Y * r.cY - r.cZ * ic);
-        double C = k1 * r.Z * r.Z + r.X * r.X + r.Y * r.Y - 2.0 * r.Z * ic;
-        double D = B * B - 4.0 * A * C;
+        const double B = k1 * r.Z * r.cZ + r.X * r.cX + r.Y * r.cY - r.cZ * ic;
+        const double C = k1 * r.Z * r.Z + r.X * r.X + r.Y * r.Y - 2.0 * r.Z * ic;
+        const double D = B * B - A * C;
         if (D < 0.0) return false;
-        double sq = fsqrt(D);
-        double sgnB = (B < 0.0) ? -1.0 : 1.0;
-        double sigma = (c > 0) ? -1.0 : 1.0;
-        double q = -0.5 * (B + sgnB * sq);
+        __asm__ volatile("");
+        const double sq = fsqrt(D);
+        const double sgnB = (B < 0.0) ? -1.0 : 1.0;
+        const double sigma = (c > 0) ? -1.0 : 1.0;
+        const double q = -(B + sgnB * sq);
         double s;
-        if (sigma == sgnB) s = (q != 0.0) ? fdiv(C, q) : fdiv(-B + sigma * sq, 2.0 * A);
+        if (sigma == sgnB) s = (q != 0.0) ? fdiv(C, q) : fdiv(-B + sigma * sq, A);
         else s = fdiv(q, A);
         r.X += s * r.cX;
         r.Y += s * r.cY;
@@ -684,7 +734,8 @@ __device__ __forceinline__ bool intersect_ray(const SD& d, Ray& r, unsigned& ite
             const double u = 1.0 + fsqrt_pos(t, irt);
             double P, Q;
             asphere_pq(d, r2, P, Q);
-            double E = c * irt + 2.0 * Q;
+            const double E = conic_factor(d, irt, Q);
+            prof.e = E;
             double dF = -E * Xi * cX - E * Yi * cY + cZ;
             if (fabs(dF) < kNewtonEps) { alive = false; break; }
             // one reciprocal for both quotients: w = 1/(u dF), 1/u = dF w,
@@ -719,11 +770,9 @@ __device__ __forceinline__ bool intersect_ray(const SD& d, Ray& r, unsigned& ite
             double Y2 = Yi * Yi;
             double t = 1.0 - K * Y2;
             double irt = rsqrt_pos(t);
-            double P, Q;
-            asphere_pq(d, Y2, P, Q);
-            double Fy = (c * Y2) * rcp_fin(1.0 + fsqrt_pos(t, irt)) + P;
+            toric_profile(d, Yi, Y2, t, irt, prof);
+            const double Fy = prof.f, dFy = prof.e;
             double F = Zi - Fy - 0.5 * cR * (Xi * Xi + Zi * Zi - Fy * Fy);
-            double dFy = c * Yi * irt + 2.0 * Q * Yi;
             double dF = -cR * Xi * cX + (cR * Fy - 1.0) * dFy * cY + (1.0 - cR * Zi) * cZ;
             if (fabs(dF) < kNewtonEps) { alive = false; break; }
             s2 = fma(-F, rcp_fin(dF), s1);
@@ -737,6 +786,12 @@ __device__ __forceinline__ bool intersect_ray(const SD& d, Ray& r, unsigned& ite
     return true;   // AuxClass
 }
 
+template <class SD>
+__device__ __forceinline__ bool intersect_ray(const SD& d, Ray& r, unsigned& iters) {
+    Profile prof;
+    return intersect_ray(d, r, iters, prof);
+}
+
 // Surface::ApplyConstrains (surface.cpp:264-321), Shade::ApplyConstrains
 // (:652-699).  The bounds (s0 * s0, -+s0/2, c0 -+ s0/2, ...) are formed once
 // on the host (D_MASK), the same IEEE values the reference forms per ray.
@@ -748,27 +803,27 @@ __device__ __forceinline__ bool mask_ray(const SD& d, double X, double Y) {
     double xr = X - c0, yr = Y - c1;
     if (type == RT_SHADE) {
         if (shape == RT_CIRCLE) return !(xr * xr + yr * yr <= p[D_MASK]);
-        return !((xr >= p[D_MASK]) && (xr <= p[D_MASK + 1]) && (yr >= p[D_MASK + 2]) && (yr <= p[D_MASK + 3]));
+        return !((xr >= p[D_MASK]) & (xr <= p[D_MASK + 1]) & (yr >= p[D_MASK + 2]) & (yr <= p[D_MASK + 3]));
     }
     if (shape == RT_CIRCLE) return !(xr * xr + yr * yr > p[D_MASK]);
-    return !((X < p[D_MASK]) || (X > p[D_MASK + 1]) || (Y < p[D_MASK + 2]) || (Y > p[D_MASK + 3]));
+    return !((X < p[D_MASK]) | (X > p[D_MASK + 1]) | (Y < p[D_MASK + 2]) | (Y > p[D_MASK + 3]));
 }
 
 // surface_reflection kernels (surface.cu:771-827)
 template <class SD>
-__device__ __forceinline__ void reflect_ray(const SD& d, Ray& r) {
+__device__ __forceinline__ void reflect_ray(const SD& d, Ray& r, const Profile* given = nullptr) {
     const int cls = d.cls();
     if (cls == RT_PLANE) { r.cZ = -r.cZ; return; }
     if (cls == RT_CONIC) {
         double dFdX, dFdY;
-        conic_derivs(d, r.X, r.Y, dFdX, dFdY);
+        conic_derivs(d, r.X, r.Y, dFdX, dFdY, given);
         double a2 = fdiv(2.0 * (r.cX * dFdX + r.cY * dFdY + r.cZ), dFdX * dFdX + dFdY * dFdY + 1.0);
         r.cX -= a2 * dFdX;
         r.cY -= a2 * dFdY;
         r.cZ -= a2;
     } else if (cls == RT_TORIC) {
         double dFdX, dFdY, dFdZ;
-        toric_derivs(d, r.X, r.Y, r.Z, dFdX, dFdY, dFdZ);
+        toric_derivs(d, r.X, r.Y, r.Z, dFdX, dFdY, dFdZ, given);
         double a2 = fdiv(2.0 * (r.cX * dFdX + r.cY * dFdY + r.cZ * dFdZ), dFdX * dFdX + dFdY * dFdY + dFdZ * dFdZ);
         r.cX -= a2 * dFdX;
         r.cY -= a2 * dFdY;
@@ -778,7 +833,7 @@ __device__ __forceinline__ void reflect_ray(const SD& d, Ray& r) {
 
 // refraction kernels (surface.cu:956-1066); false on total internal reflection
 template <class SD>
-__device__ __forceinline__ bool refract_ray(const SD& d, Ray& r, double mu) {
+__device__ __forceinline__ bool refract_ray(const SD& d, Ray& r, double mu, const Profile* given = nullptr) {
     const int cls = d.cls();
     double a, b, a2, G;
     if (cls == RT_PLANE) {
@@ -794,8 +849,8 @@ __device__ __forceinline__ bool refract_ray(const SD& d, Ray& r, double mu) {
         return true;
     }
     double dFdX, dFdY, dFdZ = 1.0;
-    if (cls == RT_CONIC) conic_derivs(d, r.X, r.Y, dFdX, dFdY);
-    else if (cls == RT_TORIC) toric_derivs(d, r.X, r.Y, r.Z, dFdX, dFdY, dFdZ);
+    if (cls == RT_CONIC) conic_derivs(d, r.X, r.Y, dFdX, dFdY, given);
+    else if (cls == RT_TORIC) toric_derivs(d, r.X, r.Y, r.Z, dFdX, dFdY, dFdZ, given);
     else return true;
     G = dFdX * dFdX + dFdY * dFdY + dFdZ * dFdZ;
     const double iG = rcp(G);
@@ -813,7 +868,7 @@ __device__ __forceinline__ bool refract_ray(const SD& d, Ray& r, double mu) {
 
 // grating kernels (surface.cu:1247-1520); false for an evanescent order
 template <class SD>
-__device__ __forceinline__ bool diffract_ray(const SD& d, Ray& r, double mu, double L) {
+__device__ __forceinline__ bool diffract_ray(const SD& d, Ray& r, double mu, double L, const Profile* given = nullptr) {
     const int cls = d.cls();
     const bool refl = (d.grtype() == RT_REFLECTIVE);
     double a, b, a2, G;
@@ -842,13 +897,13 @@ __device__ __forceinline__ bool diffract_ray(const SD& d, Ray& r, double mu, dou
     }
     double dFdX, dFdY, dFdZ = 1.0, u, v, w;
     if (cls == RT_CONIC) {
-        conic_derivs(d, r.X, r.Y, dFdX, dFdY);
+        conic_derivs(d, r.X, r.Y, dFdX, dFdY, given);
         G = fdiv(dFdX, dFdY * dFdY + 1.0);
         u = rsqrt(1.0 + dFdX * G);
         v = -dFdY * u * G;
         w = -u * G;
     } else if (cls == RT_TORIC) {
-        toric_derivs(d, r.X, r.Y, r.Z, dFdX, dFdY, dFdZ);
+        toric_derivs(d, r.X, r.Y, r.Z, dFdX, dFdY, dFdZ, given);
         G = fdiv(dFdX, dFdY * dFdY + dFdZ * dFdZ);    // D5
         u = rsqrt(1.0 + dFdX * G);
         v = -dFdY * u * G;
@@ -907,16 +962,18 @@ __device__ __forceinline__ double grating_order(const SD& d, double lam) {
 }
 
 // truncation toward zero to uint32 (ccd_coordinates_kernel, ccd.cu:30-45):
-// negative and NaN -> 0, >= 2^32 -> 0xffffffff
+// negative and NaN -> 0, >= 2^32 -> 0xffffffff, what v_cvt_u32_f64 itself does
+// (in C a conversion out of range is undefined: the instruction is named)
 __device__ __forceinline__ uint32_t trunc_u32(double v) {
-    if (!(v >= 0.0)) return 0u;
-    if (v >= 4294967296.0) return 0xffffffffu;
-    return (uint32_t)v;
+    uint32_t u;
+    __asm__("v_cvt_u32_f64 %0, %1" : "=v"(u) : "v"(v));
+    return u;
 }
 
+// v >= 0
 __device__ __forceinline__ bool near_edge(double v) {
-    double f = v - floor(v);
-    return (f < 1e-9) || (1.0 - f < 1e-9);
+    const double f = __builtin_amdgcn_fract(v);
+    return (f < 1e-9) | (1.0 - f < 1e-9);
 }
 
 // ------------------------------------------------------------ fused trace
@@ -933,7 +990,8 @@ struct BeamArg {
 struct TraceArgs {
     const double* table;          // n_surf device records of DEV_STRIDE
     const double* pool;           // device spline pool
-    int n_surf, pool_len, flags, pad;
+    int n_surf, pool_len, flags;
+    int direct;                   // stats are the caller's counters (see kStatCopies)
     BeamArg beam;
     uint64_t seed, ray_begin, n;
     double *X, *Y, *Z, *cX, *cY, *cZ, *L;
@@ -976,24 +1034,72 @@ struct TraceArgs {
     uint64_t n_groups;
 };
 constexpr int kBeamRec = (int)(sizeof(BeamArg) / sizeof(double));
-// copies of the statistics counters the trace kernels add to (TraceArgs::stats
-// points at kStatCopies x RT_STATS_LEN counters, workgroup b adding to copy
-// b % kStatCopies)
+// Copies of the statistics counters that a trace of more than kStatCopies
+// workgroups adds to (TraceArgs::stats points at kStatCopies x RT_STATS_LEN
+// counters, workgroup b adding to copy b % kStatCopies): adds to one address
+// are served one after the other, 7-10 ns each.  A smaller trace adds to the
+// caller's counters itself (TraceArgs::direct), without the fold's launch
+// (4 of the 23 us of a 256-ray trace).
 constexpr int kStatCopies = 64;
+// rays that entered dead, in a trace's own counters (not a caller's counter)
+constexpr int kStDead = 7;
 
-// stats[k] += sum of the copies' counter k, and the copies cleared for the
-// next launch (one workgroup).  The caller's counters are added to
-// atomically: traces of distinct schemes on distinct streams may fold into
-// one caller buffer at the same time.
-__device__ __forceinline__ void stats_fold_body(unsigned long long* copies, unsigned long long* stats) {
-    for (int k = threadIdx.x; k < RT_STATS_LEN; k += blockDim.x) {
+// The counters that follow from the others, in an array st in LDS: per surface
+// the rays alive on entry (those alive at the first surface less the losses
+// before it), the rays alive at the end and, when a frame was formed (ccd),
+// the hits: the rays that left a CCD surface alive less those off the frame.
+// Counted per wave they were 14 of a workgroup's 22 adds, and the atomics of
+// all workgroups are a resource that the frames need (about 25e9 a second
+// whatever they hit).  Called by every thread of the workgroup; the results
+// are there after its next barrier.
+template <class T>
+__device__ __forceinline__ void derive_counts(T* st, const double* table, int n_surf, bool ccd) {
+    const int s = (int)threadIdx.x;              // (workgroups have at least 64 lanes, schemes at most 32 surfaces)
+    if (s > n_surf) return;
+    T alive = st[RT_ST_RAYS] - st[kStDead], hits = 0;
+    for (int k = 0; k < s; ++k) {
+        alive -= st[RT_ST_SURF + 4 * k + 2] + st[RT_ST_SURF + 4 * k + 3];
+        const double* p = table + (size_t)k * DEV_STRIDE;
+        if (s == n_surf && ccd && (int)p[RT_S_TYPE] == RT_DETECTOR && p[RT_S_CCD_XDIM] > 0.0) hits += alive;
+    }
+    if (s == n_surf) {
+        st[RT_ST_GOOD] = alive;
+        if (ccd) st[RT_ST_CCD_HITS] = hits - st[RT_ST_CCD_OFFCHIP];
+    } else if ((int)table[(size_t)s * DEV_STRIDE + RT_S_TYPE] != RT_AUXTYPE) {
+        st[RT_ST_SURF + 4 * s] = alive;
+    }
+}
+
+// stats[k] += sum of the copies' counter k, with the derived counters, and the
+// copies cleared for the next launch (one workgroup of kFoldThreads).  The
+// caller's counters are added to atomically: traces of distinct schemes on
+// distinct streams may fold into one caller buffer at the same time.
+constexpr int kFoldParts = 7;
+constexpr int kFoldThreads = 1024;
+static_assert(kFoldParts * RT_STATS_LEN <= kFoldThreads, "a thread per (part, counter)");
+
+__device__ __forceinline__ void stats_fold_body(unsigned long long* copies, unsigned long long* stats,
+                                                const double* table, int n_surf, bool ccd) {
+    __shared__ unsigned long long part[kFoldParts][RT_STATS_LEN], st[RT_STATS_LEN];
+    const int g = (int)threadIdx.x / RT_STATS_LEN, k = (int)threadIdx.x % RT_STATS_LEN;
+    if (g < kFoldParts) {
         unsigned long long t = 0;
-        for (int c = 0; c < kStatCopies; ++c) {
+        for (int c = g; c < kStatCopies; c += kFoldParts) {
             t += copies[(size_t)c * RT_STATS_LEN + k];
             copies[(size_t)c * RT_STATS_LEN + k] = 0;
         }
-        if (t) atomicAdd(&stats[k], t);
+        part[g][k] = t;
     }
+    __syncthreads();
+    if (g == 0) {
+        unsigned long long t = 0;
+        for (int q = 0; q < kFoldParts; ++q) t += part[q][k];
+        st[k] = t;
+    }
+    __syncthreads();
+    derive_counts(st, table, n_surf, ccd);
+    __syncthreads();
+    if (g == 0 && k != kStDead && st[k]) atomicAdd(&stats[k], st[k]);
 }
 
 // Recording modes of the trace kernels (template argument MODE of
@@ -1033,7 +1139,8 @@ struct TraceCtx {
     unsigned* hist;
     double* flux;
     bool do_hist, do_flux;
-    unsigned n_oob, n_hit, n_off, n_edge;
+    unsigned n_rays, n_dead;      // this lane's rays, and those of them that entered dead
+    unsigned n_oob, n_off, n_edge;
     double n_prev;                // n2 of the last action (reused where the next n1 is the same table)
     unsigned last_it;             // Newton iterations of the last intersection (adjoint tape)
     uint32_t lk;                  // wavelength grid index of the current ray
@@ -1041,6 +1148,27 @@ struct TraceCtx {
 
 __device__ __forceinline__ void lds_add(unsigned* counter, unsigned v) {
     if (v) atomicAdd(counter, v);
+}
+
+// The block's counters complete: every lane's own counts added to those of its
+// waves, and added to the caller's counters or the workgroup's copy.  Called by
+// every thread of the workgroup, after its rays.
+__device__ __forceinline__ void flush_counts(const TraceCtx& c, unsigned long long* stats, bool direct,
+                                             const double* table, int n_surf) {
+    lds_add(&c.st[RT_ST_RAYS], c.n_rays);
+    lds_add(&c.st[kStDead], c.n_dead);
+    lds_add(&c.st[RT_ST_SPLINE_OOB], c.n_oob);
+    lds_add(&c.st[RT_ST_CCD_OFFCHIP], c.n_off);
+    lds_add(&c.st[RT_ST_CCD_EDGE], c.n_edge);
+    __syncthreads();
+    if (direct) {
+        derive_counts(c.st, table, n_surf, c.do_hist || c.do_flux);
+        __syncthreads();
+    } else {
+        stats += (size_t)(blockIdx.x % kStatCopies) * RT_STATS_LEN;
+    }
+    for (int k = threadIdx.x; k < RT_STATS_LEN; k += blockDim.x)
+        if (c.st[k] && !(direct && k == kStDead)) atomicAdd(&stats[k], (unsigned long long)c.st[k]);
 }
 
 // Hit counts pre-aggregated within the wave before the global atomics: the
@@ -1051,13 +1179,13 @@ __device__ __forceinline__ void lds_add(unsigned* counter, unsigned v) {
 constexpr int kPeelRounds = 8;
 
 __device__ __forceinline__ void hist_add_wave(unsigned* hist, uint32_t pix, bool on) {
-    unsigned long long pending = __ballot(on);
+    unsigned long long pending = wave_ballot(on);
     bool mine = on;
     for (int round = 0; round < kPeelRounds && pending; ++round) {
         const int leader = __ffsll((long long)pending) - 1;
         const uint32_t lp = (uint32_t)__builtin_amdgcn_readlane((int)pix, leader);
         const bool match = mine && pix == lp;
-        const unsigned long long m = __ballot(match);
+        const unsigned long long m = wave_ballot(match);
         if ((int)__lane_id() == leader) atomicAdd(&hist[lp], (unsigned)__popcll(m));
         mine = mine && !match;
         pending &= ~m;
@@ -1129,7 +1257,7 @@ template <int NV>
 __device__ __forceinline__ void ext_add(unsigned long long* e, double* b, bool on, double x, double y = 0.0) {
     bool inside = x >= b[0] && -x >= b[1];
     if (NV == 2) inside = inside && y >= b[2] && -y >= b[3];
-    if (__ballot(on && !inside) == 0) return;
+    if (wave_ballot(on && !inside) == 0) return;
     const double inf = __builtin_inf();
     const bool xon = on && x == x, yon = on && y == y;
     double t = swap_min<32>(xon ? x : inf, xon ? -x : inf);
@@ -1175,76 +1303,76 @@ __device__ __forceinline__ void surface_step(const SD& d0, int s, Ray& r, bool& 
         // only the first surface and rotated frames normalise here
         if (s == 0 || d.rot(0) || d.rot(1) || d.rot(2)) normalize_ray(r.cX, r.cY, r.cZ);
     }
-    if constexpr ((MODE & kRecExt) != 0) ext_add<1>(c.ext + s * kExtPerSurf, c.ext_bnd + s * kExtPerSurf, alive, r.cZ);   // :995
+    if constexpr ((MODE & kRecExt) != 0)                         // :995
+        ext_add<1>(c.ext + s * kExtPerSurf, c.ext_bnd + s * kExtPerSurf, alive, r.cZ);
     if (d.type() == RT_AUXTYPE) return;                          // :1000
-    unsigned long long entering = __ballot(alive);
-    if (__lane_id() == 0 && entering) atomicAdd(&c.st[RT_ST_SURF + 4 * s], (unsigned)__popcll(entering));
+    // the lanes alive here, after the intersection, past the aperture and after
+    // the action, as lane masks: a flag carried from surface to surface in a
+    // vector register costs a select and two compares each
+    const unsigned long long entering = wave_ballot(alive);
     unsigned it = 0;
-    bool lost_int = false, lost_mask = false, lost_act = false;
+    bool met = false, passed = false, out = false;
     if (alive) {
-        alive = intersect_ray(d, r, it, sink);                   // :1002
-        lost_int = !alive;
-    }
-    c.last_it = it;
-    const bool met = alive;           // alive after the intersection
-    const unsigned long long met_mask = __ballot(met);
-    bool passed = false;              // alive after the aperture mask
-    if (alive) {
-        alive = mask_ray(d, r.X, r.Y);                           // :1014
-        passed = alive;
-        lost_mask = !alive;
-        if (alive) {                                             // :1035
-            if (d.type() == RT_MIRROR) {
-                reflect_ray(d, r);
-            } else if (DERIV && (d.type() == RT_LENS || d.type() == RT_GRATING)) {
-                const double mu = lv[col];
-                if (out_of_table(mu)) {
-                    alive = false;
-                    ++c.n_oob;
-                } else if (d.type() == RT_LENS) {
-                    alive = refract_ray(d, r, mu);
-                } else {
-                    alive = diffract_ray(d, r, mu, lv[col + 1]);
-                }
-            } else if (d.type() == RT_LENS || d.type() == RT_GRATING) {
-                int e1 = 0, e2 = 0;
-                double n1, n2;
-                if (col >= 0) {
-                    int q = col;
-                    const bool t1 = !d.n1reuse() && d.n1spline();
-                    n1 = d.n1reuse() ? c.n_prev : (t1 ? lv[q++] : p[RT_S_N1VAL]);
-                    n2 = d.n2spline() ? lv[q] : p[RT_S_N2VAL];
-                    e1 = t1 && n1 != n1;
-                    e2 = d.n2spline() && n2 != n2;
-                } else {
-                    n1 = d.n1reuse() ? c.n_prev : fn_eval(c.pool, d.n1spline(), p[RT_S_N1VAL], r.lam, e1);
-                    n2 = fn_eval(c.pool, d.n2spline(), p[RT_S_N2VAL], r.lam, e2);
-                }
-                c.n_prev = n2;
-                if (e1 | e2) {
-                    alive = false;
-                    ++c.n_oob;
-                } else {
-                    // mu = n1/n2 (surface.cu:1095-1096), L = m lambda / n2 / d (:1568)
-                    const double in2 = rcp(n2);
-                    double mu = n1 * in2;
-                    if (d.type() == RT_LENS) {
-                        alive = refract_ray(d, r, mu);
+        Profile prof;
+        met = intersect_ray(d, r, it, prof, sink);               // :1002
+        if (met) {
+            passed = mask_ray(d, r.X, r.Y);                      // :1014
+            if (passed) {                                        // :1035
+                const Profile* given = has_profile(d) ? &prof : nullptr;
+                out = true;
+                if (d.type() == RT_MIRROR) {
+                    reflect_ray(d, r, given);
+                } else if (DERIV && (d.type() == RT_LENS || d.type() == RT_GRATING)) {
+                    const double mu = lv[col];
+                    if (out_of_table(mu)) {
+                        out = false;
+                        ++c.n_oob;
+                    } else if (d.type() == RT_LENS) {
+                        out = refract_ray(d, r, mu, given);
                     } else {
-                        double m = grating_order(d, r.lam);
-                        double Lg = m * r.lam * in2 * p[D_INV_D];
-                        alive = diffract_ray(d, r, mu, Lg);
+                        out = diffract_ray(d, r, mu, lv[col + 1], given);
+                    }
+                } else if (d.type() == RT_LENS || d.type() == RT_GRATING) {
+                    int e1 = 0, e2 = 0;
+                    double n1, n2;
+                    if (col >= 0) {
+                        int q = col;
+                        const bool t1 = !d.n1reuse() && d.n1spline();
+                        n1 = d.n1reuse() ? c.n_prev : (t1 ? lv[q++] : p[RT_S_N1VAL]);
+                        n2 = d.n2spline() ? lv[q] : p[RT_S_N2VAL];
+                        e1 = t1 && n1 != n1;
+                        e2 = d.n2spline() && n2 != n2;
+                    } else {
+                        n1 = d.n1reuse() ? c.n_prev : fn_eval(c.pool, d.n1spline(), p[RT_S_N1VAL], r.lam, e1);
+                        n2 = fn_eval(c.pool, d.n2spline(), p[RT_S_N2VAL], r.lam, e2);
+                    }
+                    c.n_prev = n2;
+                    if (e1 | e2) {
+                        out = false;
+                        ++c.n_oob;
+                    } else {
+                        // mu = n1/n2 (surface.cu:1095-1096), L = m lambda / n2 / d (:1568)
+                        const double in2 = rcp(n2);
+                        double mu = n1 * in2;
+                        if (d.type() == RT_LENS) {
+                            out = refract_ray(d, r, mu, given);
+                        } else {
+                            double m = grating_order(d, r.lam);
+                            double Lg = m * r.lam * in2 * p[D_INV_D];
+                            out = diffract_ray(d, r, mu, Lg, given);
+                        }
                     }
                 }
+                // :1040.  Only an action changes the direction since the entry
+                // normalisation: a stop, a Shade or a detector keeps it (the
+                // reference's renormalisation would move it by one ulp at most)
+                if (out && (d.type() == RT_MIRROR || d.type() == RT_LENS || d.type() == RT_GRATING))
+                    normalize_ray(r.cX, r.cY, r.cZ);
             }
-            // :1040.  Only an action changes the direction since the entry
-            // normalisation: a stop, a Shade or a detector keeps it (the
-            // reference's renormalisation would move it by one ulp at most)
-            if (alive && (d.type() == RT_MIRROR || d.type() == RT_LENS || d.type() == RT_GRATING))
-                normalize_ray(r.cX, r.cY, r.cZ);
-            lost_act = !alive;
         }
     }
+    c.last_it = it;
+    const unsigned long long met_mask = wave_ballot(met), out_mask = wave_ballot(out);
     if constexpr ((MODE & kRecExt) != 0) {
         // the action changes only the cosines, so X, Y are still those of
         // the intersection (:1005-1008) and of the mask (:1017-1020)
@@ -1252,20 +1380,22 @@ __device__ __forceinline__ void surface_step(const SD& d0, int s, Ray& r, bool& 
         double* b = c.ext_bnd + s * kExtPerSurf;
         ext_add<2>(e + 2, b + 2, met, r.X, r.Y);
         ext_add<2>(e + 6, b + 6, passed, r.X, r.Y);
-        ext_add<1>(e + 10, b + 10, alive, r.cZ);                 // :1042
+        ext_add<1>(e + 10, b + 10, out, r.cZ);                   // :1042
     }
     if constexpr ((MODE & kRecLoss) != 0) {
-        if (lost_int) c.loss = (unsigned char)(1 + 3 * s);
-        if (lost_mask) c.loss = (unsigned char)(2 + 3 * s);
-        if (lost_act) c.loss = (unsigned char)(3 + 3 * s);
+        if (alive && !out) c.loss = (unsigned char)((!met ? 1 : !passed ? 2 : 3) + 3 * s);
     }
+    alive = out;
     if (d.ikind() == IK_CONIC_NEWTON || d.ikind() == IK_TORIC_NEWTON) lds_add(&c.st[RT_ST_SURF + 4 * s + 1], it);
     // lost at the intersection: entered, not met; at the mask or the action:
-    // met, not alive at the end (one ballot each of the alive flag)
-    const unsigned long long li = entering & ~met_mask, la = met_mask & ~__ballot(alive);
-    if (__lane_id() == 0) {
-        if (li) atomicAdd(&c.st[RT_ST_SURF + 4 * s + 2], (unsigned)__popcll(li));
-        if (la) atomicAdd(&c.st[RT_ST_SURF + 4 * s + 3], (unsigned)__popcll(la));
+    // met, not alive at the end.  The rays alive on entry follow from these
+    // (derive_counts)
+    const unsigned long long li = entering & ~met_mask, la = met_mask & ~out_mask;
+    if (li | la) {
+        if (__lane_id() == 0) {
+            if (li) atomicAdd(&c.st[RT_ST_SURF + 4 * s + 2], (unsigned)__popcll(li));
+            if (la) atomicAdd(&c.st[RT_ST_SURF + 4 * s + 3], (unsigned)__popcll(la));
+        }
     }
     if (d.ccd() && (c.do_hist || c.do_flux)) {
         // ccd_coordinates_kernel (rt_cuda_engine_ccd.cu:30-45) with a bounds check (D10);
@@ -1281,10 +1411,9 @@ __device__ __forceinline__ void surface_step(const SD& d0, int s, Ray& r, bool& 
             double vx = (r.X + p[D_HALF_X]) * p[D_INV_XPIX];
             double vy = (r.Y + p[D_HALF_Y]) * p[D_INV_YPIX];
             uint32_t px = trunc_u32(vx), py = trunc_u32(vy);
-            on = px < xdim && py < ydim;
+            on = (px < xdim) & (py < ydim);
             if (on) {
                 pix = py * xdim + px;
-                ++c.n_hit;
                 if (near_edge(vx) || near_edge(vy)) ++c.n_edge;
                 if (DERIV && c.do_flux) {
                     const double w = lv[col];
@@ -1522,7 +1651,7 @@ __device__ __forceinline__ void trace_body(const TraceArgs& a, Surfaces surfaces
     c.flux = a.flux;
     c.do_hist = (a.flags & RT_TRACE_HIST) && a.hist;
     c.do_flux = (a.flags & RT_TRACE_FLUX) && a.flux;
-    c.n_oob = c.n_hit = c.n_off = c.n_edge = 0;
+    c.n_rays = c.n_dead = c.n_oob = c.n_off = c.n_edge = 0;
     c.n_prev = 0.0;
     const bool store = (a.flags & RT_TRACE_STORE) != 0;
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
@@ -1569,6 +1698,8 @@ __device__ __forceinline__ void trace_body(const TraceArgs& a, Surfaces surfaces
             alive = valid && ka->F[k] != 0;
         }
         if constexpr ((MODE & kRecLoss) != 0) c.loss = alive ? 0 : kLossDead;
+        c.n_rays += valid ? 1u : 0u;
+        if constexpr (BEAM < 0) c.n_dead += valid && !alive ? 1u : 0u;
         surfaces(r, alive, c, i);
         if constexpr ((MODE & kRecLoss) != 0)
             if (valid) kernel_args()->loss[i] = c.loss;
@@ -1576,39 +1707,34 @@ __device__ __forceinline__ void trace_body(const TraceArgs& a, Surfaces surfaces
             // the ray pointers are read from the argument segment where they are
             // used, not held in SGPRs across the surface chain
             const cargs ka = kernel_args();
-            if (ka->X) {
+            if (ka->X && (c.do_hist || c.do_flux)) {
+                // rows that stream past the frames: without a place in the
+                // caches they leave the frames theirs (echelle of 1e7 rays,
+                // both frames and the rays: 892 -> 880 us)
+                __builtin_nontemporal_store(r.X, &ka->X[i]);
+                __builtin_nontemporal_store(r.Y, &ka->Y[i]);
+                __builtin_nontemporal_store(r.Z, &ka->Z[i]);
+                __builtin_nontemporal_store(r.cX, &ka->cX[i]);
+                __builtin_nontemporal_store(r.cY, &ka->cY[i]);
+                __builtin_nontemporal_store(r.cZ, &ka->cZ[i]);
+                __builtin_nontemporal_store(r.lam, &ka->L[i]);
+            } else if (ka->X) {
                 ka->X[i] = r.X; ka->Y[i] = r.Y; ka->Z[i] = r.Z;
                 ka->cX[i] = r.cX; ka->cY[i] = r.cY; ka->cZ[i] = r.cZ;
                 ka->L[i] = r.lam;
             }
             if (ka->F) ka->F[i] = (signed char)alive;
         }
-        unsigned long long good = __ballot(alive), all = __ballot(valid);
-        if (__lane_id() == 0) {
-            atomicAdd(&s_stats[RT_ST_RAYS], (unsigned)__popcll(all));
-            if (good) atomicAdd(&s_stats[RT_ST_GOOD], (unsigned)__popcll(good));
-        }
         if constexpr (kTiles)
             tile_group_moments(kernel_args()->group_part, (i - threadIdx.x) / blockDim.x,
                                (a.n + blockDim.x - 1) / blockDim.x, a.ray_begin + (i - threadIdx.x), a.n_groups,
                                alive, r.X, r.Y, tile_iter++);
     }
-    lds_add(&s_stats[RT_ST_SPLINE_OOB], c.n_oob);
-    lds_add(&s_stats[RT_ST_CCD_HITS], c.n_hit);
-    lds_add(&s_stats[RT_ST_CCD_OFFCHIP], c.n_off);
-    lds_add(&s_stats[RT_ST_CCD_EDGE], c.n_edge);
-    __syncthreads();
-    if (a.stats) {
-        // one of kStatCopies copies of the counters per workgroup (folded
-        // afterwards): thousands of workgroups adding to the same few lines at
-        // the end of a launch would serialise on them
-        unsigned long long* dst = a.stats + (size_t)(blockIdx.x % kStatCopies) * RT_STATS_LEN;
-        for (int k = threadIdx.x; k < RT_STATS_LEN; k += blockDim.x)
-            if (s_stats[k]) atomicAdd(&dst[k], (unsigned long long)s_stats[k]);
-    }
+    if (a.stats) flush_counts(c, a.stats, a.direct != 0, a.table, a.n_surf);
     if constexpr ((MODE & kRecExt) != 0) {
         // a row per workgroup, reduced afterwards (atomics of every workgroup on
         // the same few lines are served one after the other)
+        __syncthreads();                             // every wave's rays are done
         for (int k = threadIdx.x; k < a.n_surf * kExtPerSurf; k += blockDim.x)
             a.ext[(size_t)k * gridDim.x + blockIdx.x] = s_ext[k];
     }
@@ -1672,7 +1798,7 @@ __device__ __forceinline__ void trace_batch_body(const TraceArgs& a, Surfaces su
     c.hist = nullptr;
     c.flux = nullptr;
     c.do_hist = c.do_flux = false;
-    c.n_oob = c.n_hit = c.n_off = c.n_edge = 0;
+    c.n_rays = c.n_dead = c.n_oob = c.n_off = c.n_edge = 0;
     c.n_prev = 0.0;
     const bool store = (a.flags & RT_TRACE_STORE) != 0;
 
@@ -1704,6 +1830,7 @@ __device__ __forceinline__ void trace_batch_body(const TraceArgs& a, Surfaces su
             ray.X = ray.Y = ray.Z = ray.cX = ray.cY = ray.lam = 0.0;
             ray.cZ = 1.0;
         }
+        c.n_rays += valid ? 1u : 0u;
         surfaces(ray, alive, c, r0 + r);
         if (store && valid) {
             const cargs kb = kernel_args();
@@ -1714,11 +1841,6 @@ __device__ __forceinline__ void trace_batch_body(const TraceArgs& a, Surfaces su
                 kb->L[g] = ray.lam;
             }
             if (kb->F) kb->F[g] = (signed char)alive;
-        }
-        unsigned long long good = __ballot(alive), all = __ballot(valid);
-        if (__lane_id() == 0) {
-            if (all) atomicAdd(&s_stats[RT_ST_RAYS], (unsigned)__popcll(all));
-            if (good) atomicAdd(&s_stats[RT_ST_GOOD], (unsigned)__popcll(good));
         }
         // spot moments of the tile (asked for): count and means, then
         // squared deviations
@@ -1739,16 +1861,7 @@ __device__ __forceinline__ void trace_batch_body(const TraceArgs& a, Surfaces su
             tile_group_moments(a.group_part, t, a.n_tiles, (t - ts[inst]) * blockDim.x, a.n_groups, alive, ray.X,
                                ray.Y, tile_iter++);
     }
-    lds_add(&s_stats[RT_ST_SPLINE_OOB], c.n_oob);
-    __syncthreads();
-    if (a.stats) {
-        // one of kStatCopies copies of the counters per workgroup (folded
-        // afterwards): thousands of workgroups adding to the same few lines at
-        // the end of a launch would serialise on them
-        unsigned long long* dst = a.stats + (size_t)(blockIdx.x % kStatCopies) * RT_STATS_LEN;
-        for (int k = threadIdx.x; k < RT_STATS_LEN; k += blockDim.x)
-            if (s_stats[k]) atomicAdd(&dst[k], (unsigned long long)s_stats[k]);
-    }
+    if (a.stats) flush_counts(c, a.stats, a.direct != 0, a.table, a.n_surf);
 }
 
 }  // namespace rt

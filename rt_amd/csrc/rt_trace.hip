@@ -527,6 +527,7 @@ struct rt_hip_scheme {
     int block = rt::kBlock;          // lanes per workgroup
     int waves = 7;                   // minimum waves per SIMD asked of the compiler (0: its choice)
     int grid_mult = 16;              // persistent workgroups per CU = grid_mult x resident ones
+    bool launch_given = false;       // set by the caller or the autotuner: taken as it is
     // surface unroll depth: 1, the whole chain unrolled (the generated
     // kernel); 0, a runtime loop over the records (the generic kernel)
     int unroll = 1;
@@ -728,8 +729,10 @@ __global__ __launch_bounds__(256) void rt_ltab_kernel(rt::LtabArgs a) { rt::ltab
 
 __global__ __launch_bounds__(256) void rt_dtab_kernel(rt::DtabArgs a) { rt::dtab_body(a); }
 
-__global__ __launch_bounds__(256) void rt_stats_fold_kernel(unsigned long long* copies, unsigned long long* stats) {
-    rt::stats_fold_body(copies, stats);
+__global__ __launch_bounds__(rt::kFoldThreads) void rt_stats_fold_kernel(unsigned long long* copies,
+                                                                         unsigned long long* stats,
+                                                                         const double* table, int n_surf, int ccd) {
+    rt::stats_fold_body(copies, stats, table, n_surf, ccd != 0);
 }
 
 namespace {
@@ -766,9 +769,19 @@ int stat_copies_alloc(unsigned long long** p) {
     return RT_OK;
 }
 
-// stats += the copies (cleared), on `st` after the trace
-int stats_fold(unsigned long long* copies, unsigned long long* stats, hipStream_t st) {
-    hipLaunchKernelGGL(rt_stats_fold_kernel, dim3(1), dim3(256), 0, st, copies, stats);
+// where a trace of `grid` workgroups adds its counters: the caller's, or the copies
+void stats_target(TraceArgs& a, unsigned long long* copies, unsigned long long* stats, unsigned grid) {
+    a.direct = stats && grid <= (unsigned)rt::kStatCopies ? 1 : 0;
+    a.stats = !stats ? nullptr : a.direct ? stats : copies;
+}
+
+// stats += the copies (cleared), on `st` after the trace `a`, unless it added
+// to them itself
+int stats_fold(const TraceArgs& a, unsigned long long* stats, hipStream_t st) {
+    if (!stats || a.direct) return RT_OK;
+    const int ccd = ((a.flags & RT_TRACE_HIST) && a.hist) || ((a.flags & RT_TRACE_FLUX) && a.flux);
+    hipLaunchKernelGGL(rt_stats_fold_kernel, dim3(1), dim3(rt::kFoldThreads), 0, st, a.stats, stats, a.table, a.n_surf,
+                       ccd);
     HIP_TRY(hipGetLastError(), RT_ERR_FAILED);
     return RT_OK;
 }
@@ -952,6 +965,21 @@ static void beam_uniforms(TraceArgs& a) {
 }
 
 namespace {
+// The launch of a trace of a scheme whose launch nobody has set: the defaults,
+// but 8 waves per SIMD for rays given by the caller (their kernel waits on its
+// loads and on splines in LDS: 1e6 echelle rays 121 -> 112 us) and, where both
+// frames take an atomic of every ray and bound the trace, workgroups of 512
+// lanes from 2^20 rays on (1e7 echelle rays 926 -> 892 us; with fewer rays, or
+// one frame or none, 256 lanes are as fast or faster).
+void trace_shape(const rt_hip_scheme* sch, bool gen, const TraceArgs& a, int rec, int& block, int& waves) {
+    block = sch->block;
+    waves = sch->waves;
+    if (sch->launch_given || rec) return;
+    if (!gen) waves = 8;
+    const bool frames = (a.flags & RT_TRACE_HIST) && a.hist && (a.flags & RT_TRACE_FLUX) && a.flux;
+    if (gen && frames && a.n >= (1u << 20)) block = 512;
+}
+
 // The workgroups of a recording trace with extents: as many as are resident
 // at once and no more, so that each walks many rays under bounds it has met
 // (ext_add) and leaves one row of keys, in whole rounds of rays.
@@ -999,7 +1027,6 @@ int trace_launch(const rt_hip_scheme* sch, const double* beam_desc, uint64_t see
     a.n = n_rays;
     a.X = X; a.Y = Y; a.Z = Z; a.cX = cX; a.cY = cY; a.cZ = cZ; a.L = lambda; a.F = flag;
     a.hist = ccd_hist; a.flux = ccd_flux; a.dump = dump; a.dump_flag = dump_flag;
-    a.stats = stats ? sch->stat_copies : nullptr;
     a.loss = loss;
     a.group_part = group_part;
     a.n_groups = n_groups;
@@ -1011,6 +1038,8 @@ int trace_launch(const rt_hip_scheme* sch, const double* beam_desc, uint64_t see
 
     const uint64_t nk = gen && sch->unroll ? dtab_nk(sch->dt, beam_desc) : 0;
     unsigned grid = 0;
+    int block, waves;
+    trace_shape(sch, gen, a, rec, block, waves);
     // the rows of extents keys of as many workgroups as this launch can have
     auto ext_rows = [&](uint64_t most) {
         const int r = sch->work.ensure(WorkBufs::EXT_KEYS,
@@ -1024,21 +1053,23 @@ int trace_launch(const rt_hip_scheme* sch, const double* beam_desc, uint64_t see
                            (dump ? RT_JIT_VAR_DUMP : 0) | ((rec & rt::kRecLoss) ? RT_JIT_VAR_LOSS : 0) |
                                ((rec & rt::kRecExt) ? RT_JIT_VAR_EXT : 0) |
                                ((rec & rt::kRecSpots) ? RT_JIT_VAR_SPOTS : 0),
-                           sch->block, sch->waves, sch->device);
+                           block, waves, sch->device);
     if (fn) {
         if (nk) {
             rc = dtab_fill(sch->dt, a, sch->table_dev, sch->pool_dev, sch->n_surf, nk, st);
             if (rc != RT_OK) return rc;
             a.ltab = sch->dt.tab_dev;
             a.lt_nk = nk;
+            a.pool_len = 0;                            // every function comes from the table
+            lds = 0;
         }
         // persistent grid: the workgroups that are resident at once on every CU
         // (from the compiled kernel's registers and LDS), times grid_mult
         int resident = 0;
-        if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&resident, fn, sch->block, lds) != hipSuccess ||
+        if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&resident, fn, block, lds) != hipSuccess ||
             resident < 1)
             resident = 1;
-        uint64_t want = (n_rays + sch->block - 1) / sch->block;
+        uint64_t want = (n_rays + block - 1) / block;
         uint64_t cap = (uint64_t)cus * resident * sch->grid_mult;
         grid = (unsigned)(want < cap ? want : cap);
         if (extents) {
@@ -1046,14 +1077,15 @@ int trace_launch(const rt_hip_scheme* sch, const double* beam_desc, uint64_t see
             rc = ext_rows((uint64_t)cus * resident);
             if (rc != RT_OK) return rc;
         }
+        stats_target(a, sch->stat_copies, stats, grid);
         void* params[] = {&a};
-        HIP_TRY(hipModuleLaunchKernel(fn, grid, 1, 1, sch->block, 1, 1, (unsigned)lds, st, params, nullptr),
+        HIP_TRY(hipModuleLaunchKernel(fn, grid, 1, 1, block, 1, 1, (unsigned)lds, st, params, nullptr),
                 RT_ERR_FAILED);
         g_last_kernel = "generated";
-        if (block_used) *block_used = sch->block;
+        if (block_used) *block_used = block;
         if (getenv("RT_HIP_VERBOSE"))
             fprintf(stderr, "rt_hip: trace generated kernel %p, %zu rays, block %d, waves %d, grid %u, table %llu, "
-                            "record %d\n", (void*)fn, n_rays, sch->block, sch->waves, grid, (unsigned long long)nk,
+                            "record %d\n", (void*)fn, n_rays, block, waves, grid, (unsigned long long)nk,
                     rec);
     } else {
         uint64_t want = (n_rays + kBlock - 1) / kBlock;
@@ -1076,6 +1108,7 @@ int trace_launch(const rt_hip_scheme* sch, const double* beam_desc, uint64_t see
                                 : beam_mode == RT_BEAM_CONIC  ? rt_trace_kernel<RT_BEAM_CONIC, R>
                                 : beam_mode == RT_BEAM_GAUSS  ? rt_trace_kernel<RT_BEAM_GAUSS, R>
                                                               : rt_trace_kernel<kLoad, R>);
+        stats_target(a, sch->stat_copies, stats, grid);
         hipLaunchKernelGGL(kern, dim3(grid), dim3(kBlock), lds, st, a);
         g_last_kernel = "generic";
         if (block_used) *block_used = kBlock;
@@ -1088,8 +1121,7 @@ int trace_launch(const rt_hip_scheme* sch, const double* beam_desc, uint64_t see
                            (const unsigned long long*)a.ext, grid, extents);
         HIP_TRY(hipGetLastError(), RT_ERR_FAILED);
     }
-    if (stats) return stats_fold(sch->stat_copies, stats, st);
-    return RT_OK;
+    return stats_fold(a, stats, st);
 }
 }  // namespace
 
@@ -1166,6 +1198,7 @@ extern "C" int rt_hip_scheme_set_launch(rt_hip_scheme* sch, int block, int waves
     sch->block = block;
     sch->waves = waves;
     sch->grid_mult = grid_mult;
+    sch->launch_given = true;
     return RT_OK;
 }
 
@@ -1247,6 +1280,8 @@ extern "C" int rt_hip_autotune(rt_hip_scheme* sch, const double* beam_desc, uint
     struct Cand { int b, w, m; float ms; int regs, local, u; };
     std::vector<Cand> cands;
     const int bb0 = sch->block, bw0 = sch->waves, bm0 = sch->grid_mult, bu0 = sch->unroll;
+    const bool given0 = sch->launch_given;
+    sch->launch_given = true;
     // mean time of `reps` back-to-back launches of candidate c
     auto timed = [&](const Cand& c, int reps, float& ms) -> int {
         sch->block = c.b; sch->waves = c.w; sch->grid_mult = c.m; sch->unroll = c.u;
@@ -1355,6 +1390,7 @@ extern "C" int rt_hip_autotune(rt_hip_scheme* sch, const double* beam_desc, uint
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     sch->block = bb; sch->waves = bw; sch->grid_mult = bm; sch->unroll = bu;
+    if (rc != RT_OK) sch->launch_given = given0;
     if (rc != RT_OK) return rc;
     if (best_ms) *best_ms = best;
     return RT_OK;
@@ -1649,7 +1685,6 @@ int batch_trace(const rt_hip_batch* bc, const double* beam_desc, uint64_t seed, 
     if (flags & RT_TRACE_STORE) {
         a.X = X; a.Y = Y; a.Z = Z; a.cX = cX; a.cY = cY; a.cZ = cZ; a.L = lambda; a.F = flag;
     }
-    a.stats = stats ? b->stat_copies : nullptr;
     a.tile_start = b->tile_start_dev;
     a.tile_inst = b->tile_inst_dev;
     a.ray_start = b->ray_start_dev;
@@ -1661,7 +1696,7 @@ int batch_trace(const rt_hip_batch* bc, const double* beam_desc, uint64_t seed, 
     a.inst_stride = (uint64_t)b->n_surf * rt::DEV_STRIDE;
 
     const int cus = rt_device_cus();
-    const size_t lds = b->pool_len * sizeof(double);
+    size_t lds = b->pool_len * sizeof(double);
     hipStream_t st = (hipStream_t)stream;
     const int beam_mode = (int)a.beam.v[RT_B_TYPE];
     if (b->beams_on) {
@@ -1681,6 +1716,8 @@ int batch_trace(const rt_hip_batch* bc, const double* beam_desc, uint64_t seed, 
             if (rc != RT_OK) return rc;
             a.ltab = b->lt.tab_dev;
             a.lt_nk = nk;
+            a.pool_len = 0;                            // every function comes from the table
+            lds = 0;
         }
         int resident = 0;
         if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&resident, fn, b->block, lds) != hipSuccess ||
@@ -1688,6 +1725,7 @@ int batch_trace(const rt_hip_batch* bc, const double* beam_desc, uint64_t seed, 
             resident = 1;
         uint64_t cap = (uint64_t)cus * resident * b->grid_mult;
         unsigned grid = (unsigned)(b->n_tiles < cap ? b->n_tiles : cap);
+        stats_target(a, b->stat_copies, stats, grid);
         void* params[] = {&a};
         HIP_TRY(hipModuleLaunchKernel(fn, grid, 1, 1, b->block, 1, 1, (unsigned)lds, st, params, nullptr),
                 RT_ERR_FAILED);
@@ -1708,14 +1746,13 @@ int batch_trace(const rt_hip_batch* bc, const double* beam_desc, uint64_t seed, 
         auto kern = beam_mode == RT_BEAM_PARALLEL ? rt_trace_batch_kernel<RT_BEAM_PARALLEL>
                   : beam_mode == RT_BEAM_CONIC    ? rt_trace_batch_kernel<RT_BEAM_CONIC>
                                                   : rt_trace_batch_kernel<RT_BEAM_GAUSS>;
+        stats_target(a, b->stat_copies, stats, grid);
         hipLaunchKernelGGL(kern, dim3(grid), dim3(kBlock), lds, st, a);
         g_last_kernel = "generic";
     }
     HIP_TRY(hipGetLastError(), RT_ERR_FAILED);
-    if (stats) {
-        rc = stats_fold(b->stat_copies, stats, st);
-        if (rc != RT_OK) return rc;
-    }
+    rc = stats_fold(a, stats, st);
+    if (rc != RT_OK) return rc;
     if (spots) {
         hipLaunchKernelGGL(rt_batch_spots_kernel, dim3((unsigned)b->n_inst), dim3(kInstSpotThreads), 0, st,
                            (const double*)b->moments_dev, (const uint64_t*)b->tile_start_dev, (uint64_t)b->n_inst,
