@@ -369,7 +369,8 @@ static std::string generate_adjoint_source(const std::string& sig, int beam_type
     }
     os << "    },\n"
        << "    [&](const rt::Ray& r, rt::adj::St& ad, rt::TraceCtx& c, const rt::adj::LaneRows& t, "
-          "auto& g, bool ok) -> bool {\n";
+          "auto& g, bool ok) -> bool {\n"
+       << "      rt::adj::St after = {r.X, r.Y, r.Z, r.cX, r.cY, r.cZ};\n";
     if (use_tab) os << "      double lb[" << nc << "];\n";
     for (int s = n_surf - 1; s >= 0; --s) {
         if (derived && use_tab) {
@@ -382,8 +383,8 @@ static std::string generate_adjoint_source(const std::string& sig, int beam_type
                     tab_s = true;
                 }
             os << " double gp[rt::adj::PG_N]; const bool use = rt::adj::bwd_step_d<true>(" << types[s]
-               << "{c.table + " << s << " * rt::DEV_STRIDE}, r, ad, c, t, " << k0[s] << ", gp, lb, "
-               << (tab_s ? col_base[(size_t)s] : -1) << ") && ok;";
+               << "{c.table + " << s << " * rt::DEV_STRIDE}, ad, t, " << k0[s] << ", gp, lb, "
+               << (tab_s ? col_base[(size_t)s] : -1) << ", &after) && ok;";
             for (size_t gi = 0; gi < groups.size(); ++gi) {
                 if (groups[gi].surf != s) continue;
                 os << " g.template add4<" << gi << ">(";
@@ -408,7 +409,8 @@ static std::string generate_adjoint_source(const std::string& sig, int beam_type
            << s << " * rt::DEV_STRIDE}, r, ad, c, t, " << k0[s] << ", gp";
         if (tab_s) os << ", lb, " << n1col[(size_t)s] << ", " << n2col[(size_t)s];
         else if (use_tab) os << ", lb, -1, -1";
-        os << ") && ok;";
+        else os << ", nullptr, -1, -1";
+        os << ", &after) && ok;";
         for (size_t gi = 0; gi < groups.size(); ++gi) {
             if (groups[gi].surf != s) continue;
             os << " g.template add4<" << gi << ">(";

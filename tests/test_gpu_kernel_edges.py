@@ -5,6 +5,8 @@ import numpy as np
 import pytest
 import torch
 
+from rt_amd import scheme as S
+
 pytestmark = pytest.mark.gpu
 
 
@@ -48,7 +50,7 @@ def test_group_spots_at_chunk_edges(hip, n, G):
 @pytest.mark.parametrize("n", [1, 64, 1023, 1024, 1025, 512 * 1024 + 1])
 def test_mask_counts_and_flags(hip, n):
     print(f"[mask] n={n}", flush=True)
-    from rt_amd import scheme as S
+
     g = torch.Generator().manual_seed(n)
     xy = torch.randn((2, n), generator=g, dtype=torch.float64)
     if n > 64:
@@ -162,3 +164,72 @@ def test_recorded_extents_equal_dumped_states(hip, n):
             want = (v.min(), v.max()) if v.size else (np.nan, np.nan)
             assert np.array_equal(e[s, 2 * q:2 * q + 2], want, equal_nan=True), (s, q)
     ds.close()
+
+
+def every_surface_kind():
+    """a lens, a rotated auxiliary frame, a rotated stop, an aspheric and a
+    toric lens, a plane lens face, both kinds of grating, a spherical and a
+    toric mirror, a detector: every branch of the reverse step"""
+    s = [S.Surface(S.RT_CONIC, S.RT_LENS, S.RT_CIRCLE, params=(1 / 400.0, -0.3, 0), size=(40.0, 0.0),
+                   distance=(0.1, -0.2, 20.0), angles=(0.3, -0.2, 0.0), n1=1.0, n2=1.5),
+         S.Surface(S.RT_PLANE, S.RT_AUXTYPE, distance=(0.0, 0.1, 3.0), angles=(0.0, 0.5, 1.0)),
+         S.Surface(S.RT_PLANE, S.RT_STOP, S.RT_CIRCLE, size=(40.0, 0.0), distance=(0.0, 0.0, 2.0),
+                   angles=(0.2, 0.0, 0.4)),
+         S.Surface(S.RT_PLANE, S.RT_LENS, S.RT_CIRCLE, size=(40.0, 0.0), distance=(0.0, 0.0, 5.0),
+                   angles=(0.0, 1.0, 0.0), n1=1.5, n2=1.0),
+         S.Surface(S.RT_CONIC, S.RT_LENS, S.RT_CIRCLE, params=(-1 / 300.0, 0.2, 3, 1e-6, 1e-9, 1e-13),
+                   size=(40.0, 0.0), distance=(0.0, 0.0, 10.0), n1=1.0, n2=1.6),
+         S.Surface(S.RT_TORIC, S.RT_LENS, S.RT_CIRCLE, params=(1 / 500.0, 0.1, 1, 1e-7, 1 / 350.0),
+                   size=(40.0, 0.0), distance=(0.2, 0.0, 6.0), n1=1.6, n2=1.0),
+         S.Surface(S.RT_PLANE, S.RT_GRATING, S.RT_CIRCLE, size=(60.0, 0.0), distance=(0.0, 0.0, 30.0),
+                   angles=(2.0, 0.0, 0.0), grating_type=S.RT_TRANSPARENT, order=1, gr_const=10.0),
+         S.Surface(S.RT_CONIC, S.RT_MIRROR, S.RT_CIRCLE, params=(-1 / 900.0, 0.0, 0), size=(90.0, 0.0),
+                   distance=(0.0, 0.0, 60.0), angles=(3.0, 0.0, 0.0)),
+         S.Surface(S.RT_TORIC, S.RT_MIRROR, S.RT_CIRCLE, params=(1 / 1200.0, 0.0, 0, 1 / 1500.0),
+                   size=(120.0, 0.0), distance=(0.0, 0.0, -70.0), angles=(0.0, 1.0, 0.0)),
+         S.Surface(S.RT_PLANE, S.RT_GRATING, S.RT_CIRCLE, size=(150.0, 0.0), distance=(0.0, 0.0, 80.0),
+                   grating_type=S.RT_REFLECTIVE, order=-1, gr_const=20.0),
+         S.Surface(S.RT_PLANE, S.RT_DETECTOR, S.RT_RECTANGLE, size=(400.0, 400.0), distance=(0.0, 0.0, -90.0),
+                   angles=(0.5, 0.2, 0.0), ccd=dict(xdim=64, ydim=64, xpix=5.0, ypix=5.0))]
+    return s
+
+
+@pytest.mark.parametrize("n", [1, 65, 600])
+@pytest.mark.parametrize("beam", ["conic", "parallel"])
+def test_generated_adjoint_equals_the_generic_one(hip, n, beam):
+    # the generated reverse step reads the state after each surface from the
+    # tape where the generic one replays it: the same derivatives, to the sums'
+    # and the directions' rounding (1e-11 of the largest, as for batches)
+    kind = S.RT_BEAM_CONIC if beam == "conic" else S.RT_BEAM_PARALLEL
+    b = S.Beam(type=kind, shape=S.RT_CIRCLE, params=(n, 0.0, 6.0, 1.0, 2.0), range=(0.5, 0.6), nlambda=1)
+    surf = every_surface_kind()
+    sch = S.Scheme(surf, b, name="kinds")
+    ps, pf = [], []
+    for i, q in enumerate(surf):
+        fields = [S.S_DIST + k for k in range(3)] + [S.S_ANG + k for k in range(3)]
+        if q.cls != S.RT_PLANE:
+            fields += [S.S_C, S.S_K] + [S.S_A + k for k in range(int(q.params[2]))]
+        if q.cls == S.RT_TORIC:
+            fields.append(S.S_CR)
+        if q.type == S.RT_GRATING:
+            fields.append(S.S_GRCONST)
+        ps += [i] * len(fields)
+        pf += fields
+    G = 3
+    rng = np.random.default_rng(3)
+    seeds = torch.from_numpy(rng.normal(size=(G, 3))).cuda()
+    out = []
+    for jit in (True, False):
+        prev = hip.set_jit(jit)
+        try:
+            ds = hip.DeviceScheme(sch)
+            st = torch.zeros(S.STATS_LEN, dtype=torch.int64, device="cuda")
+            out.append(ds.adjoint(seeds, ps, pf, seed=11, n=n, stats=st).cpu().numpy())
+            st = st.cpu().numpy()
+            assert st[S.ST_GOOD] == n and st[S.ST_ADJ_SKIP] == 0
+            ds.close()
+        finally:
+            hip.set_jit(prev)
+    scale = float(np.max(np.abs(out[1])))
+    assert scale > 0 and np.all(np.isfinite(out[0]))
+    assert np.all(np.abs(out[0] - out[1]) <= 1e-11 * scale), float(np.max(np.abs(out[0] - out[1]))) / scale
