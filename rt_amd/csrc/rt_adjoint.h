@@ -207,12 +207,12 @@ struct Conic {
 template <class Rec>
 RT_HD Conic conic_at(const Rec& d, double x) {
     const auto p = d.p;
-    const double c = p[RT_S_C], k1 = p[RT_S_K] + 1.0;
+    const double c = p[RT_S_C];
     Conic o;
 #if defined(__HIP_DEVICE_COMPILE__)
     const double K = p[D_K1C2];        // (k+1) c c
 #else
-    const double K = k1 * c * c;
+    const double K = (p[RT_S_K] + 1.0) * c * c;
 #endif
     const double t = 1.0 - K * x;
     const double rq = drsqrt(t);               // 1/q
@@ -313,7 +313,8 @@ constexpr int kMaxNewtonAdj = 8;    // iterations differentiated exactly (the lo
 struct NewtonSeq {
     int n;                          // iterations of the forward pass
     double s0;
-    double s[kMaxNewtonAdj];        // s^(0) .. s^(n-1); the point is at s^(n-1)
+    double s[kMaxNewtonAdj];        // s^(0) .. s^(n-2), where the steps are taken
+    double last;                    // s^(n-1), the point's
 };
 
 // The point at parameter s along the ray, the profile there, and F and
@@ -404,6 +405,7 @@ RT_UNROLL
         }
         if (!done) return false;            // more iterations than are differentiated here
         q.n = it;
+        q.last = s1;
         const double u = s1 + q.s0;
         out.X = in.X + u * in.cX; out.Y = in.Y + u * in.cY; out.Z = s1 * in.cZ;
         return true;
@@ -505,12 +507,11 @@ RT_HD void adj_intersect(const Rec& d, const St& in, const St& out, const Newton
     } else if (kind == AK_CONIC_NEWTON || kind == AK_TORIC_NEWTON) {
         double as = 0.0, as0 = 0.0;
         const int n = q.n;
+        // the returned point, at the last iterate evaluated
+        point_adj(in, q.s0, q.last, a.X, a.Y, a.Z, ain, as, as0);
 RT_UNROLL
-        for (int k = kMaxNewtonAdj - 1; k >= 0; --k) {
-            if (k == n - 1) {
-                // the returned point, at the last iterate evaluated
-                point_adj(in, q.s0, q.s[k], a.X, a.Y, a.Z, ain, as, as0);
-            } else if (k < n - 1) {
+        for (int k = kMaxNewtonAdj - 2; k >= 0; --k) {
+            if (k < n - 1) {
                 // s^(k+1) = s^(k) - F/G at s^(k)
                 const NewtonAt o = newton_at(d, kind, in, q.s0, q.s[k]);
                 const double iG = drcp(o.G);
@@ -776,7 +777,8 @@ RT_HD bool surface_adjoint(const Rec& d, const St& entry, int n_fwd, double mu, 
 namespace rt {
 namespace adj {
 
-constexpr int kTape = 7;                 // X Y Z cX cY cZ, Newton iterations
+constexpr int kTapeLanes = 256;          // lanes of the adjoint kernels' workgroups
+constexpr int kTape = 7;                 // X Y Z cX cY cZ, Newton iterations (generic kernels)
 
 struct AdjArgs {
     double beam[kBeamRec];               // beam fields + BeamUniform (first: kernarg offset 0)
@@ -786,7 +788,7 @@ struct AdjArgs {
     uint64_t seed, n, n_groups;
     const double* seeds;                 // n_groups x 3: ax, ay, b
     const int* prow;                     // n_surf x PG_N: the caller's index of (surface, slot), or -1
-    double* tape;                        // (n_surf * kTape) x lanes
+    double* tape;                        // tape_rows x lanes
     double* gacc;                        // n_par x waves (single scheme); tile-wave x n_par (batch)
     unsigned long long* stats;
     // batched adjoint (adjoint_batch_body): instance i owns records
@@ -804,8 +806,8 @@ struct AdjArgs {
     // batched adjoint with a beam per instance: n_inst records of
     // kBeamRec doubles (beam fields, then the uniform values), or null
     const double* inst_beams;
-    // rows of the tape per lane: kTape per surface, and kMaxNewtonAdj more per
-    // iterating intersection where the forward records its Newton iterates
+    // rows of the tape in memory per lane: kTape per surface in the generic
+    // kernels, the rows that are not in LDS in the generated ones (Tape)
     uint64_t tape_rows;
 };
 
@@ -871,48 +873,90 @@ __device__ __forceinline__ LaneRows lane_rows(double* base, uint64_t rows, uint6
     return b;
 }
 
+// One lane's tape.  The surface steps number its rows logically, and Map::row
+// places them: row r >= 0 is row r of LDS below NL and row r - NL of memory
+// from there; kRowZero holds 0 and kRowShared - r is row r of the surface
+// before, neither of them written; at a Newton count's row stands its number,
+// and counts lie in registers, 4 bits each.  The tape is written and read once
+// per ray at a rate near the memory's: as 7 rows per surface and all iterates
+// in memory the echelle's adjoint moved 88 rows each way, 1.4 kB a ray at 5.1
+// TB/s.  The workgroups that the registers let a CU hold leave LDS for NL = 25
+// rows of their lanes, and without the rows that are known 48 to 52 remain:
+// the kernel 268 -> 239 us at 1e6 rays and, 256 instances together, 9.5 -> 8.0 ms.
+struct PlainMap {
+    __device__ static int row(int k) { return k; }
+};
+constexpr int kRowZero = -1, kRowShared = -2;
+
+template <class Map = PlainMap, int NL = 0, int NW = 0>
+struct Tape {
+    LaneRows mem;
+    double* lds;                         // the lane's first LDS row; rows are kTapeLanes doubles apart
+    uint32_t nits[NW > 0 ? NW : 1];
+    __device__ double ld(int k) const {
+        int r = Map::row(k);
+        if (r == kRowZero) return 0.0;
+        if (r <= kRowShared) r = kRowShared - r;
+        return r < NL ? lds[r * kTapeLanes] : mem.ld(r - NL);
+    }
+    __device__ void st(int k, double v) const {
+        const int r = Map::row(k);
+        if (r < 0) return;
+        if (r < NL) lds[r * kTapeLanes] = v;
+        else mem.st(r - NL, v);
+    }
+    // the i-th of consecutive rows in memory from k on, i a run-time value
+    __device__ void st_mem(int k, int i, double v) const { mem.st(Map::row(k) - NL + i, v); }
+    __device__ void put_count(int k, unsigned n) {
+        const int j = Map::row(k);
+        nits[j / 8] |= (n < 15u ? n : 15u) << (4 * (j % 8));
+    }
+    __device__ int count(int k) const {
+        const int j = Map::row(k);
+        return (int)((nits[j / 8] >> (4 * (j % 8))) & 15u);
+    }
+};
+
+template <class T>
+__device__ __forceinline__ T make_tape(const AdjArgs& a, double* lds, uint64_t G, uint64_t lane) {
+    T t;
+    t.mem = lane_rows(a.tape, a.tape_rows, G, lane);
+    t.lds = lds + threadIdx.x;
+RT_UNROLL
+    for (uint32_t& w : t.nits) w = 0;
+    return t;
+}
+
 // forward through one surface: tape of the entry state (rows k0 .. k0+6),
 // the trace's surface step, the Newton count
 // (lv, col: the ray's per-wavelength table values, as surface_step takes them)
 // (DERIV: lv holds the derived table's columns, as surface_step takes them;
-// ITER: an iterating intersection records its first kMaxNewtonAdj Newton
-// iterates in rows k0 + kTape ..)
+// ITER, the generated kernels: an iterating intersection records its Newton
+// iterates in rows k0 + kTape ..: not s^(0), which is 0, nor s^(7), the last
+// that is differentiated and so the point's)
+template <class T>
 struct TapeIterSink {
-    const LaneRows* t;
+    const T* t;
     int k0;
     __device__ void operator()(unsigned k, double s) const {
-        if (k < (unsigned)kMaxNewtonAdj) t->st(k0 + kTape + (int)k, s);
+        if (k >= 1 && k < (unsigned)kMaxNewtonAdj - 1) t->st_mem(k0 + kTape + 1, (int)k - 1, s);
     }
 };
 
-template <bool DERIV = false, bool ITER = false, class SD>
-__device__ __forceinline__ void fwd_step(const SD& d, int s, Ray& r, bool& alive, TraceCtx& c, const LaneRows& t,
-                                         int k0, const double* lv = nullptr, int col = -1) {
+template <bool DERIV = false, bool ITER = false, class SD, class T>
+__device__ __forceinline__ void fwd_step(const SD& d, int s, Ray& r, bool& alive, TraceCtx& c, T& t, int k0,
+                                         const double* lv = nullptr, int col = -1) {
     if (alive) {
         t.st(k0 + 0, r.X); t.st(k0 + 1, r.Y); t.st(k0 + 2, r.Z);
         t.st(k0 + 3, r.cX); t.st(k0 + 4, r.cY); t.st(k0 + 5, r.cZ);
     }
-    if constexpr (ITER) surface_step<SD, 0, DERIV>(d, s, r, alive, c, lv, col, TapeIterSink{&t, k0});
+    if constexpr (ITER) surface_step<SD, 0, DERIV>(d, s, r, alive, c, lv, col, TapeIterSink<T>{&t, k0});
     else surface_step<SD, 0, DERIV>(d, s, r, alive, c, lv, col);
     // the Newton count (row 6) only where the intersection iterates
-    if ((d.ikind() == IK_CONIC_NEWTON || d.ikind() == IK_TORIC_NEWTON) && alive) t.st(k0 + 6, (double)c.last_it);
-}
-
-// backward through one surface: gp receives the surface's parameter
-// derivatives (zero where the replay fails).  false: no adjoint (curved
-// grating, replay lost).  The lanes of the wave are converged again when it
-// returns, so the caller can reduce gp across the wave.  With lv (the ray's
-// per-wavelength table values), n1 and n2 are lv[n1col] and lv[n2col], or
-// the surface's constants where a column is -1.
-// the Newton iterates the forward step recorded (fwd_step with ITER)
-template <class SD>
-__device__ __forceinline__ NewtonSeq taped_iterates(const SD&, const LaneRows& t, int k0, int nit) {
-    NewtonSeq q;
-    q.n = nit;
-    q.s0 = 0.0;
-RT_UNROLL
-    for (int k = 0; k < kMaxNewtonAdj; ++k) q.s[k] = k < nit ? t.ld(k0 + kTape + k) : 0.0;
-    return q;
+    if (d.ikind() == IK_CONIC_NEWTON || d.ikind() == IK_TORIC_NEWTON) {
+        if constexpr (ITER) t.put_count(k0 + 6, alive ? c.last_it : 0u);
+        else if (alive) t.st(k0 + 6, (double)c.last_it);
+    }
 }
 
 #if defined(__clang__)
@@ -927,14 +971,14 @@ RT_UNROLL
 // the projection a - u (u . a); it is taken after each action only: a
 // component of a along the direction passes the intersections, frame changes
 // and stops before that action unchanged, adds to no parameter (a rotation
-// moves the direction across itself) and is projected out there.  An
-// iterating surface takes its iterates (given).  Measured on the echelle's 48
+// moves the direction across itself) and is projected out there.  q: the
+// count and the iterates before the last of an iterating surface.  Measured on the echelle's 48
 // derivatives at 1e6 rays: 5,460 vector instructions per 64 rays where
 // surface_adjoint took 7,040, 153 registers where it took 168 and spilled, and
 // the kernel 316 -> 268 us.
 template <class Rec>
 __device__ __forceinline__ bool surface_adjoint_after(const Rec& d, const St& entry, const St& after, double mu,
-                                                      double L, St& a, double* gp, const NewtonSeq& given) {
+                                                      double L, St& a, double* gp, NewtonSeq& q) {
     const auto p = d.p;
     const int type = d.type(), kind = d.ikind();
     St sT = entry;
@@ -943,10 +987,11 @@ __device__ __forceinline__ bool surface_adjoint_after(const Rec& d, const St& en
         adj_transform(d, sT, a, gp);
         return true;
     }
-    NewtonSeq q = given;
     if (kind == AK_CONIC_NEWTON || kind == AK_TORIC_NEWTON) {
-        if (given.n < 1 || given.n > kMaxNewtonAdj) return false;   // more are not differentiated here
-        q.s0 = -sT.Z * drcp(sT.cZ);
+        if (q.n < 1 || q.n > kMaxNewtonAdj) return false;   // more are not differentiated here
+        const double icZ = drcp(sT.cZ);
+        q.s0 = -sT.Z * icZ;
+        q.last = after.Z * icZ;                             // Z = s cZ
     }
     const St sI = {after.X, after.Y, after.Z, sT.cX, sT.cY, sT.cZ};
     const bool acts = type == RT_MIRROR || type == RT_LENS || type == RT_GRATING;
@@ -969,30 +1014,41 @@ __device__ __forceinline__ bool surface_adjoint_after(const Rec& d, const St& en
 #pragma clang fp contract(on)
 #endif
 
+// backward through one surface: gp receives the surface's parameter
+// derivatives (to be left out where it returns false: no adjoint, a curved
+// grating or a lost replay).  The lanes of the wave are converged again when
+// it returns, so the caller can reduce gp across the wave.  With lv (the ray's
+// per-wavelength table values), n1 and n2 are lv[n1col] and lv[n2col], or
+// the surface's constants where a column is -1.
 // ITER: the forward recorded its Newton iterates and `after` holds the state
 // after the surface; it becomes the entry state.
-template <bool ITER, class SD>
-__device__ __forceinline__ bool bwd_surface(const SD& d, St& ad, const LaneRows& t, int k0, double* gp, double mu,
-                                            double L, St* after) {
+template <bool ITER, class SD, class T>
+__device__ __forceinline__ bool bwd_surface(const SD& d, St& ad, const T& t, int k0, double* gp, double mu, double L,
+                                            St* after) {
 RT_UNROLL
     for (int k = 0; k < PG_N; ++k) gp[k] = 0.0;
     const St entry = {t.ld(k0 + 0), t.ld(k0 + 1), t.ld(k0 + 2), t.ld(k0 + 3), t.ld(k0 + 4), t.ld(k0 + 5)};
-    const int nit = (d.ikind() == IK_CONIC_NEWTON || d.ikind() == IK_TORIC_NEWTON) ? (int)t.ld(k0 + 6) : 0;
+    const bool iterates = d.ikind() == IK_CONIC_NEWTON || d.ikind() == IK_TORIC_NEWTON;
     if constexpr (ITER) {
         NewtonSeq q;
         q.n = 0;
-        if (nit != 0) q = taped_iterates(d, t, k0, nit);
+        q.s0 = q.last = q.s[0] = 0.0;
+        if (iterates) {
+            q.n = t.count(k0 + 6);
+RT_UNROLL
+            for (int k = 1; k < kMaxNewtonAdj - 1; ++k) q.s[k] = k < q.n - 1 ? t.ld(k0 + kTape + k) : 0.0;
+        }
         const bool ok = surface_adjoint_after(d, entry, *after, mu, L, ad, gp, q);
         *after = entry;
         return ok;
     }
-    return surface_adjoint(d, entry, nit, mu, L, ad, gp);
+    return surface_adjoint(d, entry, iterates ? (int)t.ld(k0 + 6) : 0, mu, L, ad, gp);
 }
 
-template <bool ITER = false, class SD>
-__device__ __forceinline__ bool bwd_step(const SD& d, const Ray& r, St& ad, const TraceCtx& c, const LaneRows& t,
-                                         int k0, double* gp, const double* lv = nullptr, int n1col = -1,
-                                         int n2col = -1, St* after = nullptr) {
+template <bool ITER = false, class SD, class T>
+__device__ __forceinline__ bool bwd_step(const SD& d, const Ray& r, St& ad, const TraceCtx& c, const T& t, int k0,
+                                         double* gp, const double* lv = nullptr, int n1col = -1, int n2col = -1,
+                                         St* after = nullptr) {
     const auto p = d.p;
     // mu and L exactly as the forward pass formed them
     double mu = 0.0, L = 0.0;
@@ -1015,9 +1071,9 @@ __device__ __forceinline__ bool bwd_step(const SD& d, const Ray& r, St& ad, cons
 
 // bwd_step for kernels reading the derived table: mu = lv[col] and, for a
 // grating, L = lv[col + 1], the values the forward step read
-template <bool ITER = false, class SD>
-__device__ __forceinline__ bool bwd_step_d(const SD& d, St& ad, const LaneRows& t, int k0, double* gp,
-                                           const double* lv, int col, St* after) {
+template <bool ITER = false, class SD, class T>
+__device__ __forceinline__ bool bwd_step_d(const SD& d, St& ad, const T& t, int k0, double* gp, const double* lv,
+                                           int col, St* after) {
     double mu = 0.0, L = 0.0;
     if (d.type() == RT_LENS || d.type() == RT_GRATING) {
         mu = lv[col];
@@ -1127,13 +1183,13 @@ RT_UNROLL
 };
 
 // forward(r, alive, c, tape); backward(r, ad, c, tape, acc, ok) -> ok, with
-// tape the lane's rows of a.tape (n_surf * kTape rows of G lanes) and acc the
+// tape the lane's rows (a.tape: a.tape_rows rows of G lanes) and acc the
 // wave's accumulators in a.gacc (n_par rows of G / 64 waves).  The ray loop is
 // wave-uniform (a wave's lanes take rays i0 .. i0 + 63 together and lanes past
 // the end run masked), so that the backward steps can reduce across the wave;
 // lanes whose ray is lost or whose replay fails compute on and are masked out
 // of the sums.  The tape size must fit a buffer resource (checked by the host).
-template <int BEAM, class Acc, class Fwd, class Bwd>
+template <int BEAM, class Acc, class T = Tape<>, class Fwd, class Bwd>
 __device__ __forceinline__ void adjoint_body(const AdjArgs& a, Fwd forward, Bwd backward) {
     extern __shared__ double s_pool[];
     __shared__ unsigned s_stats[RT_STATS_LEN];
@@ -1171,12 +1227,13 @@ __device__ __forceinline__ void adjoint_body(const AdjArgs& a, Fwd forward, Bwd 
         c.lk = (uint32_t)jl;
         bool alive = in;
         c.n_rays += in ? 1u : 0u;
-        forward(r, alive, c, lane_rows(a.tape, a.tape_rows, G, lane));
+        T tape = make_tape<T>(a, s_pool, G, lane);
+        forward(r, alive, c, tape);
         if (!wave_ballot(alive)) continue;                        // wave-uniform
         const uint64_t g = i % a.n_groups;
         const double bx = a.seeds[3 * g], by = a.seeds[3 * g + 1], b = a.seeds[3 * g + 2];
         St ad = {bx + b * r.X, by + b * r.Y, 0.0, 0.0, 0.0, 0.0};
-        const bool ok = backward(r, ad, c, lane_rows(a.tape, a.tape_rows, G, lane), acc, alive);
+        const bool ok = backward(r, ad, c, tape, acc, alive);
         if (alive && !ok) ++skipped;
     }
     acc.end(a, wave, W, lw);
@@ -1191,7 +1248,7 @@ __device__ __forceinline__ void adjoint_body(const AdjArgs& a, Fwd forward, Bwd 
 // tile-wave go to a.gacc[(tile * waves_per_group + wave) * n_par + j] and are
 // reduced per instance afterwards.  Every wave runs the backward (lanes
 // without a live ray masked), so every slot is written.
-template <int BEAM, class Acc, class Fwd, class Bwd>
+template <int BEAM, class Acc, class T = Tape<>, class Fwd, class Bwd>
 __device__ __forceinline__ void adjoint_batch_body(const AdjArgs& a, Fwd forward, Bwd backward) {
     extern __shared__ double s_pool[];
     __shared__ unsigned s_stats[RT_STATS_LEN];
@@ -1243,13 +1300,14 @@ __device__ __forceinline__ void adjoint_batch_body(const AdjArgs& a, Fwd forward
         c.lk = (uint32_t)jl;
         bool alive = in;
         c.n_rays += in ? 1u : 0u;
-        forward(ray, alive, c, lane_rows(a.tape, a.tape_rows, G, lane));
+        T tape = make_tape<T>(a, s_pool, G, lane);
+        forward(ray, alive, c, tape);
         const uint64_t g = r % ka->n_groups;
         const double* sd = ka->seeds + (inst * ka->n_groups + g) * 3;
         const double bx = sd[0], by = sd[1], b = sd[2];
         St ad = {bx + b * ray.X, by + b * ray.Y, 0.0, 0.0, 0.0, 0.0};
         acc.tile_begin(a, t * wpg + wib, lw, a.n_tiles * wpg);
-        const bool ok = backward(ray, ad, c, lane_rows(a.tape, a.tape_rows, G, lane), acc, alive);
+        const bool ok = backward(ray, ad, c, tape, acc, alive);
         if (alive && !ok) ++skipped;
         acc.tile_end(a, t * wpg + wib, lw);
     }

@@ -30,7 +30,7 @@ using rt::adj::kTape;
 
 namespace {
 
-constexpr int kAdjBlock = 256;
+constexpr int kAdjBlock = rt::adj::kTapeLanes;
 
 // p[0 .. n) = 0 by a kernel (a caller may capture the call in a hipGraph,
 // where memset nodes are avoided)
@@ -48,14 +48,13 @@ constexpr int kReduceChunks = 64;        // first-stage workgroups per parameter
 
 template <int BEAM>
 __global__ __launch_bounds__(kAdjBlock) void rt_adjoint_kernel(AdjArgs a) {
-    using rt::adj::LaneRows;
     rt::adj::adjoint_body<BEAM, rt::adj::WaveAcc>(
         a,
-        [&](Ray& r, bool& alive, rt::TraceCtx& c, const LaneRows& t) {
+        [&](Ray& r, bool& alive, rt::TraceCtx& c, const rt::adj::Tape<>& t) {
             for (int s = 0; s < a.n_surf; ++s)
                 rt::adj::fwd_step(rt::DynSurf{c.table + (size_t)s * rt::DEV_STRIDE}, s, r, alive, c, t, s * kTape);
         },
-        [&](const Ray& r, rt::adj::St& ad, rt::TraceCtx& c, const LaneRows& t, const auto& g, bool ok) {
+        [&](const Ray& r, rt::adj::St& ad, rt::TraceCtx& c, const rt::adj::Tape<>& t, const auto& g, bool ok) {
             for (int s = a.n_surf - 1; s >= 0; --s) {
                 // the row table is uniform: read through the constant address space
                 const __attribute__((address_space(4))) int* rows =
@@ -78,14 +77,13 @@ __global__ __launch_bounds__(kAdjBlock) void rt_adjoint_kernel(AdjArgs a) {
 // the same surface steps over a batch's tiles (adjoint_batch_body)
 template <int BEAM>
 __global__ __launch_bounds__(kAdjBlock) void rt_adjoint_batch_kernel(AdjArgs a) {
-    using rt::adj::LaneRows;
     rt::adj::adjoint_batch_body<BEAM, rt::adj::TileOut>(
         a,
-        [&](Ray& r, bool& alive, rt::TraceCtx& c, const LaneRows& t) {
+        [&](Ray& r, bool& alive, rt::TraceCtx& c, const rt::adj::Tape<>& t) {
             for (int s = 0; s < a.n_surf; ++s)
                 rt::adj::fwd_step(rt::DynSurf{c.table + (size_t)s * rt::DEV_STRIDE}, s, r, alive, c, t, s * kTape);
         },
-        [&](const Ray& r, rt::adj::St& ad, rt::TraceCtx& c, const LaneRows& t, const auto& g, bool ok) {
+        [&](const Ray& r, rt::adj::St& ad, rt::TraceCtx& c, const rt::adj::Tape<>& t, const auto& g, bool ok) {
             for (int s = a.n_surf - 1; s >= 0; --s) {
                 // the row table is uniform: read through the constant address space
                 const __attribute__((address_space(4))) int* rows =
@@ -275,6 +273,16 @@ int adjoint_waves() {
     return w ? atoi(w) : 3;
 }
 
+// Tape rows that the lanes of a generated kernel keep in LDS: as many as leave
+// a CU the workgroups that its registers let in (one wave per SIMD each; 160 kB
+// of LDS, handed out in blocks of 1280 bytes, and 1 kB of counters a
+// workgroup), at most 25.  A kernel that stages the spline pool keeps none.
+int adjoint_lds_rows(int waves, size_t pool_bytes) {
+    if (pool_bytes) return 0;
+    const int w = waves > 0 ? waves : 1;
+    return std::min(25, (160 * 1024 / w - 2 * 1280) / (int)(kAdjBlock * sizeof(double)));
+}
+
 // workgroups launched per resident slot (the persistent grid is CUs x
 // resident x this, within the tape's 2 GiB buffer): 16 for batches, where the
 // hardware's dealing of the extra workgroups balances instances of uneven
@@ -327,26 +335,29 @@ extern "C" int rt_hip_adjoint(const rt_hip_scheme* sch, const double* beam_desc,
     // the kernel generated for this structure and parameter list, else the generic one
     // (grid-wavelength beams: the generated kernel reads the per-wavelength table)
     const uint64_t nk = rt_scheme_dtab_nk(sch, beam_desc);
+    const int waves = adjoint_waves();
+    // the table's kernels read no spline
+    const size_t pool_bytes = pool_len * sizeof(double);
+    const int lds_rows = adjoint_lds_rows(waves, nk ? 0 : pool_bytes);
     hipFunction_t fn = nullptr;
     if (rt_jit_enabled())
-        fn = rt_jit_adjoint_kernel(rt_scheme_signature(sch), beam_type, host, n_surf, kAdjBlock, adjoint_waves(),
-                                   rt_scheme_device(sch), false, nk != 0);
+        fn = rt_jit_adjoint_kernel(rt_scheme_signature(sch), beam_type, host, n_surf, kAdjBlock, waves,
+                                   rt_scheme_device(sch), false, nk != 0, lds_rows);
     auto kern = beam_type == RT_BEAM_PARALLEL ? rt_adjoint_kernel<RT_BEAM_PARALLEL>
               : beam_type == RT_BEAM_CONIC    ? rt_adjoint_kernel<RT_BEAM_CONIC>
                                               : rt_adjoint_kernel<RT_BEAM_GAUSS>;
-    // the table's kernels read no spline
-    const size_t lds = fn && nk ? 0 : pool_len * sizeof(double);
-    if (fn && nk) a.pool_len = 0;
+    const size_t lds = fn && lds_rows ? (size_t)lds_rows * kAdjBlock * sizeof(double) : pool_bytes;
+    if (fn && lds_rows) a.pool_len = 0;
     int resident = 0;
     hipError_t oe = fn ? hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&resident, fn, kAdjBlock, lds)
                        : hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, kern, kAdjBlock, lds);
     if (oe != hipSuccess || resident < 1) resident = 1;
     uint64_t want = (n_rays + kAdjBlock - 1) / kAdjBlock;
     uint64_t cap = (uint64_t)rt_device_cus() * resident * adjoint_grid_mult(1);
-    // the tape (tape_rows rows: n_surf * kTape, plus the Newton iterates the
-    // generated kernel records) and the accumulators (n_params rows) of G
+    // the tape (tape_rows rows: n_surf * kTape, or those of a generated kernel
+    // that are not in LDS) and the accumulators (n_params rows) of G
     // lanes are addressed as buffer resources of at most 2^31 - 1 bytes
-    a.tape_rows = fn ? (uint64_t)rt_jit_adjoint_tape_rows(rt_scheme_signature(sch)) : (uint64_t)n_surf * kTape;
+    a.tape_rows = fn ? (uint64_t)rt_jit_adjoint_tape_rows(rt_scheme_signature(sch), lds_rows) : (uint64_t)n_surf * kTape;
     const uint64_t rows_max = std::max<uint64_t>(a.tape_rows, (uint64_t)std::max(n_params, 1));
     const uint64_t lanes_max = 0x7fffffffull / (rows_max * sizeof(double));
     if (cap > lanes_max / kAdjBlock) cap = lanes_max / kAdjBlock;
@@ -436,22 +447,25 @@ extern "C" int rt_hip_batch_adjoint(const rt_hip_batch* b, const double* beam_de
     }
 
     const uint64_t nk = rt_batch_ltab_nk(b, beam_desc);
+    const int waves = adjoint_waves();
+    // the table's kernels read no spline
+    const size_t pool_bytes = v.pool_len * sizeof(double);
+    const int lds_rows = adjoint_lds_rows(waves, nk ? 0 : pool_bytes);
     hipFunction_t fn = nullptr;
     if (rt_jit_enabled())
-        fn = rt_jit_adjoint_kernel(*v.signature, beam_type, host, v.n_surf, kAdjBlock, adjoint_waves(), v.device,
-                                   true, nk != 0);
+        fn = rt_jit_adjoint_kernel(*v.signature, beam_type, host, v.n_surf, kAdjBlock, waves, v.device, true,
+                                   nk != 0, lds_rows);
     auto kern = beam_type == RT_BEAM_PARALLEL ? rt_adjoint_batch_kernel<RT_BEAM_PARALLEL>
               : beam_type == RT_BEAM_CONIC    ? rt_adjoint_batch_kernel<RT_BEAM_CONIC>
                                               : rt_adjoint_batch_kernel<RT_BEAM_GAUSS>;
-    // the table's kernels read no spline
-    const size_t lds = fn && nk ? 0 : v.pool_len * sizeof(double);
-    if (fn && nk) a.pool_len = 0;
+    const size_t lds = fn && lds_rows ? (size_t)lds_rows * kAdjBlock * sizeof(double) : pool_bytes;
+    if (fn && lds_rows) a.pool_len = 0;
     int resident = 0;
     hipError_t oe = fn ? hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&resident, fn, kAdjBlock, lds)
                        : hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, kern, kAdjBlock, lds);
     if (oe != hipSuccess || resident < 1) resident = 1;
     uint64_t cap = (uint64_t)rt_device_cus() * resident * adjoint_grid_mult(16);
-    a.tape_rows = fn ? (uint64_t)rt_jit_adjoint_tape_rows(*v.signature) : (uint64_t)v.n_surf * kTape;
+    a.tape_rows = fn ? (uint64_t)rt_jit_adjoint_tape_rows(*v.signature, lds_rows) : (uint64_t)v.n_surf * kTape;
     const uint64_t lanes_max = 0x7fffffffull / (a.tape_rows * sizeof(double));
     if (cap > lanes_max / kAdjBlock) cap = lanes_max / kAdjBlock;
     const unsigned grid = (unsigned)(v.n_tiles < cap ? v.n_tiles : cap);

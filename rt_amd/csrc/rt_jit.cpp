@@ -252,35 +252,75 @@ static int sig_arg(const std::string& t, int n) {
     return q == std::string::npos ? 0 : atoi(t.c_str() + q);
 }
 
-// Tape rows of one surface in the generated adjoints: kTape, plus the Newton
-// iterates the forward records where the intersection iterates (StatSurf's
-// IK, its 7th template argument)
-static int adjoint_tape_rows_of(const std::string& type) {
-    const int ik = sig_arg(type, 6);
-    return rt::adj::kTape + ((ik == rt::IK_CONIC_NEWTON || ik == rt::IK_TORIC_NEWTON) ? rt::adj::kMaxNewtonAdj : 0);
-}
-
-int rt_jit_adjoint_tape_rows(const std::string& sig) {
-    int rows = 0;
+static std::vector<std::string> sig_types(const std::string& sig) {
+    std::vector<std::string> types;
     size_t pos = 0;
     while (pos < sig.size()) {
         const size_t end = sig.find(';', pos);
-        rows += adjoint_tape_rows_of(sig.substr(pos, end - pos));
+        types.push_back(sig.substr(pos, end - pos));
         pos = end + 1;
     }
-    return rows;
+    return types;
+}
+
+// Tape of a generated adjoint kernel.  The surface steps number its rows
+// logically, k0[s] ..: the entry state (6), the Newton count, and
+// kMaxNewtonAdj iterates where the intersection iterates.  map gives each
+// logical row's place (rt::adj::Tape): the rows of the entry states come
+// first, and the first of them lie in LDS, then the iterates' rows.  Left out:
+// the Z after a plane surface, which is 0, and the direction after a surface
+// that keeps it, where that surface's own entry direction is its direction too
+// (no rotation, and not the first surface, which normalises the beam's): the
+// rows of that surface are read again.
+struct AdjTape {
+    std::vector<int> k0, map;
+    int state = 0, total = 0, counts = 0;
+};
+
+static AdjTape adjoint_tape(const std::vector<std::string>& types) {
+    using rt::adj::kTape;
+    using rt::adj::kMaxNewtonAdj;
+    AdjTape t;
+    std::vector<char> iterates;
+    for (size_t s = 0; s < types.size(); ++s) {
+        const int k = (int)t.map.size(), ik = sig_arg(types[s], 6);
+        const int before = s ? sig_arg(types[s - 1], 1) : -1;
+        iterates.push_back(ik == rt::IK_CONIC_NEWTON || ik == rt::IK_TORIC_NEWTON);
+        t.k0.push_back(k);
+        t.map.push_back(t.state++);
+        t.map.push_back(t.state++);
+        const bool flat = s && before != RT_AUXTYPE && sig_arg(types[s - 1], 6) == rt::IK_PLANE;
+        t.map.push_back(flat ? rt::adj::kRowZero : t.state++);
+        const bool kept = s > 1 && before != RT_MIRROR && before != RT_LENS && before != RT_GRATING &&
+                          sig_arg(types[s - 1], 8) == 0;
+        for (int q = 3; q < 6; ++q) {
+            if (!kept) {
+                t.map.push_back(t.state++);
+                continue;
+            }
+            const int from = t.map[(size_t)t.k0[s - 1] + q];
+            t.map.push_back(from <= rt::adj::kRowShared ? from : rt::adj::kRowShared - from);
+        }
+        t.map.push_back(iterates[s] ? t.counts++ : -1);
+        if (iterates[s]) t.map.resize(t.map.size() + kMaxNewtonAdj, -1);
+    }
+    t.total = t.state;
+    // s^(0) is 0 and the last iterate is the point's: s^(1) .. s^(kMaxNewtonAdj - 2)
+    for (size_t s = 0; s < types.size(); ++s)
+        if (iterates[s])
+            for (int k = 1; k < kMaxNewtonAdj - 1; ++k) t.map[(size_t)t.k0[s] + kTape + k] = t.total++;
+    return t;
+}
+
+int rt_jit_adjoint_tape_rows(const std::string& sig, int lds_rows) {
+    const AdjTape t = adjoint_tape(sig_types(sig));
+    return std::max(1, t.total - std::min(lds_rows, t.state));
 }
 
 static std::string generate_adjoint_source(const std::string& sig, int beam_type, const std::vector<int>& rows,
                                            int n_surf, int block, int waves = 0, bool batch = false,
-                                           bool ltab = false) {
-    std::vector<std::string> types;
-    size_t pos = 0;
-    while (pos < sig.size()) {
-        size_t end = sig.find(';', pos);
-        types.push_back(sig.substr(pos, end - pos));
-        pos = end + 1;
-    }
+                                           bool ltab = false, int lds_rows = 0) {
+    const std::vector<std::string> types = sig_types(sig);
     // per-wavelength table (RT_JIT_LTAB).  One scheme: the derived table, whose
     // mu and grating columns the forward steps read as the trace does and the
     // backward steps read again (the detector's flux weight is not read: no
@@ -334,6 +374,12 @@ static std::string generate_adjoint_source(const std::string& sig, int beam_type
     for (size_t gi = 0; gi < groups.size(); ++gi)
         for (int k = 0; k < 4; ++k)
             if (groups[gi].par[k] >= 0) map[(gi / 16) * 64 + 16 * kRowOf[k] + gi % 16] = groups[gi].par[k];
+    const AdjTape tape = adjoint_tape(types);
+    const std::vector<int>& k0 = tape.k0;
+    std::ostringstream tt;
+    tt << "rt::adj::Tape<RtTapeMap, " << std::min(lds_rows, tape.state) << ", " << std::max(1, (tape.counts + 7) / 8)
+       << ">";
+    const std::string tape_type = tt.str();
     std::ostringstream os;
     const size_t nc = col_surf.size();
     os << "#include \"rt_adjoint.h\"\n"
@@ -341,17 +387,17 @@ static std::string generate_adjoint_source(const std::string& sig, int beam_type
     for (size_t k = 0; k < map.size(); ++k) os << (k ? "," : "") << map[k];
     os << "};\n"
        << "struct RtAdjMap { __device__ static int slot(int k) { return rt_adj_slot_map[k]; } };\n"
+       << "constexpr int rt_adj_tape_map[" << tape.map.size() << "] = {";
+    for (size_t k = 0; k < tape.map.size(); ++k) os << (k ? "," : "") << tape.map[k];
+    os << "};\n"
+       << "struct RtTapeMap { __device__ static constexpr int row(int k) { return rt_adj_tape_map[k]; } };\n"
        << "extern \"C\" __global__ __launch_bounds__(" << block;
     if (waves > 0) os << ", " << waves;
     os << ") void rt_adjoint_jit(rt::adj::AdjArgs a) {\n"
        << "  rt::adj::" << (batch ? "adjoint_batch_body<" : "adjoint_body<") << beam_type
-       << ", rt::adj::GroupAcc<" << n_reg << ", RtAdjMap>>(a,\n"
-       << "    [&](rt::Ray& r, bool& alive, rt::TraceCtx& c, const rt::adj::LaneRows& t) {\n";
+       << ", rt::adj::GroupAcc<" << n_reg << ", RtAdjMap>, " << tape_type << ">(a,\n"
+       << "    [&](rt::Ray& r, bool& alive, rt::TraceCtx& c, " << tape_type << "& t) {\n";
     if (use_tab) os << "      double lv[" << nc << "];\n";
-    // tape rows of each surface: the entry state and Newton count (kTape),
-    // and the Newton iterates where the intersection iterates
-    std::vector<int> k0(n_surf, 0);
-    for (int s = 1; s < n_surf; ++s) k0[s] = k0[s - 1] + adjoint_tape_rows_of(types[s - 1]);
     for (int s = 0; s < n_surf; ++s) {
         // refractive-index columns only: the adjoint accumulates no flux, so
         // the detector's QE and spectrum are never read
@@ -368,7 +414,7 @@ static std::string generate_adjoint_source(const std::string& sig, int beam_type
         os << ");\n";
     }
     os << "    },\n"
-       << "    [&](const rt::Ray& r, rt::adj::St& ad, rt::TraceCtx& c, const rt::adj::LaneRows& t, "
+       << "    [&](const rt::Ray& r, rt::adj::St& ad, rt::TraceCtx& c, const " << tape_type << "& t, "
           "auto& g, bool ok) -> bool {\n"
        << "      rt::adj::St after = {r.X, r.Y, r.Z, r.cX, r.cY, r.cZ};\n";
     if (use_tab) os << "      double lb[" << nc << "];\n";
@@ -511,10 +557,10 @@ hipFunction_t rt_jit_kernel(const std::string& sig, int beam_mode, int variant, 
 }
 
 hipFunction_t rt_jit_adjoint_kernel(const std::string& sig, int beam_type, const std::vector<int>& rows, int n_surf,
-                                    int block, int waves, int device, bool batch, bool ltab) {
+                                    int block, int waves, int device, bool batch, bool ltab, int lds_rows) {
     std::ostringstream key;
     key << device << "|adjoint|" << (batch ? "batch|" : "") << (ltab ? "ltab|" : "") << beam_type << "|" << block
-        << "|" << waves << "|";
+        << "|" << waves << "|" << lds_rows << "|";
     for (size_t k = 0; k < rows.size(); ++k)
         if (rows[k] >= 0) key << k << ":" << rows[k] << ",";
     key << "|" << sig;
@@ -522,7 +568,7 @@ hipFunction_t rt_jit_adjoint_kernel(const std::string& sig, int beam_type, const
     Entry& e = g_cache[key.str()];
     if (e.fn) return e.fn;
     if (e.failed) return nullptr;
-    if (!compile(generate_adjoint_source(sig, beam_type, rows, n_surf, block, waves, batch, ltab), e,
+    if (!compile(generate_adjoint_source(sig, beam_type, rows, n_surf, block, waves, batch, ltab, lds_rows), e,
                  "rt_adjoint_jit")) {
         e.failed = true;
         fprintf(stderr, "rt_hip: generated adjoint kernel failed to build, using the generic kernel:\n%s\n",
