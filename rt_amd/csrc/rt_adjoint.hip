@@ -265,7 +265,7 @@ void fill_beam(AdjArgs& a, const double* beam_desc) {
 
 // minimum waves per SIMD asked of the generated kernels' register allocation:
 // 3 (168 VGPRs) measured fastest on the echelle's 48 parameters (a loss and its
-// gradient at 1e6 rays 360 us, 64 instances 12.1 ms; at 4, which spills 32
+// gradient at 1e6 rays 360 us, 256 instances 12.1 ms; at 4, which spills 32
 // registers, 380 us and 13.3 ms); RT_HIP_ADJOINT_WAVES overrides (0: the
 // compiler's choice)
 int adjoint_waves() {
