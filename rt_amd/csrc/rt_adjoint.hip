@@ -187,9 +187,7 @@ struct AdjBufs {
 int adj_buffers(WorkBufs* w, size_t tape, size_t gacc, size_t part, const std::vector<int>& rows, bool upload_rows,
                 AdjBufs& out) {
     std::vector<int>& rows_key = w->params_key;
-    int rc = w->ensure(WorkBufs::TAPE, tape * sizeof(double));
-    if (rc == RT_OK) rc = w->ensure(WorkBufs::GACC, gacc * sizeof(double));
-    if (rc == RT_OK && part) rc = w->ensure(WorkBufs::PART, part * sizeof(double));
+    int rc = w->ensure(WorkBufs::TAPE, (tape + gacc + part) * sizeof(double));
     if (rc != RT_OK) return rc;
     if (upload_rows && (rows != rows_key || !w->p[WorkBufs::PARAMS])) {
         rows_key.clear();
@@ -202,8 +200,8 @@ int adj_buffers(WorkBufs* w, size_t tape, size_t gacc, size_t part, const std::v
         rows_key = rows;
     }
     out.tape = w->get<double>(WorkBufs::TAPE);
-    out.gacc = w->get<double>(WorkBufs::GACC);
-    out.part = w->get<double>(WorkBufs::PART);
+    out.gacc = out.tape + tape;
+    out.part = out.gacc + gacc;
     out.params = w->get<int>(WorkBufs::PARAMS);
     return RT_OK;
 }
@@ -340,9 +338,10 @@ extern "C" int rt_hip_adjoint(const rt_hip_scheme* sch, const double* beam_desc,
     const size_t pool_bytes = pool_len * sizeof(double);
     const int lds_rows = adjoint_lds_rows(waves, nk ? 0 : pool_bytes);
     hipFunction_t fn = nullptr;
+    int jit_rows = 0;
     if (rt_jit_enabled())
         fn = rt_jit_adjoint_kernel(rt_scheme_signature(sch), beam_type, host, n_surf, kAdjBlock, waves,
-                                   rt_scheme_device(sch), false, nk != 0, lds_rows);
+                                   rt_scheme_device(sch), false, nk != 0, lds_rows, &jit_rows);
     auto kern = beam_type == RT_BEAM_PARALLEL ? rt_adjoint_kernel<RT_BEAM_PARALLEL>
               : beam_type == RT_BEAM_CONIC    ? rt_adjoint_kernel<RT_BEAM_CONIC>
                                               : rt_adjoint_kernel<RT_BEAM_GAUSS>;
@@ -357,7 +356,7 @@ extern "C" int rt_hip_adjoint(const rt_hip_scheme* sch, const double* beam_desc,
     // the tape (tape_rows rows: n_surf * kTape, or those of a generated kernel
     // that are not in LDS) and the accumulators (n_params rows) of G
     // lanes are addressed as buffer resources of at most 2^31 - 1 bytes
-    a.tape_rows = fn ? (uint64_t)rt_jit_adjoint_tape_rows(rt_scheme_signature(sch), lds_rows) : (uint64_t)n_surf * kTape;
+    a.tape_rows = fn ? (uint64_t)jit_rows : (uint64_t)n_surf * kTape;
     const uint64_t rows_max = std::max<uint64_t>(a.tape_rows, (uint64_t)std::max(n_params, 1));
     const uint64_t lanes_max = 0x7fffffffull / (rows_max * sizeof(double));
     if (cap > lanes_max / kAdjBlock) cap = lanes_max / kAdjBlock;
@@ -452,9 +451,10 @@ extern "C" int rt_hip_batch_adjoint(const rt_hip_batch* b, const double* beam_de
     const size_t pool_bytes = v.pool_len * sizeof(double);
     const int lds_rows = adjoint_lds_rows(waves, nk ? 0 : pool_bytes);
     hipFunction_t fn = nullptr;
+    int jit_rows = 0;
     if (rt_jit_enabled())
         fn = rt_jit_adjoint_kernel(*v.signature, beam_type, host, v.n_surf, kAdjBlock, waves, v.device, true,
-                                   nk != 0, lds_rows);
+                                   nk != 0, lds_rows, &jit_rows);
     auto kern = beam_type == RT_BEAM_PARALLEL ? rt_adjoint_batch_kernel<RT_BEAM_PARALLEL>
               : beam_type == RT_BEAM_CONIC    ? rt_adjoint_batch_kernel<RT_BEAM_CONIC>
                                               : rt_adjoint_batch_kernel<RT_BEAM_GAUSS>;
@@ -465,7 +465,7 @@ extern "C" int rt_hip_batch_adjoint(const rt_hip_batch* b, const double* beam_de
                        : hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, kern, kAdjBlock, lds);
     if (oe != hipSuccess || resident < 1) resident = 1;
     uint64_t cap = (uint64_t)rt_device_cus() * resident * adjoint_grid_mult(16);
-    a.tape_rows = fn ? (uint64_t)rt_jit_adjoint_tape_rows(*v.signature, lds_rows) : (uint64_t)v.n_surf * kTape;
+    a.tape_rows = fn ? (uint64_t)jit_rows : (uint64_t)v.n_surf * kTape;
     const uint64_t lanes_max = 0x7fffffffull / (a.tape_rows * sizeof(double));
     if (cap > lanes_max / kAdjBlock) cap = lanes_max / kAdjBlock;
     const unsigned grid = (unsigned)(v.n_tiles < cap ? v.n_tiles : cap);

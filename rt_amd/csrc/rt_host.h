@@ -26,7 +26,7 @@ int rt_set_error(int code, const char* fmt, ...) __attribute__((format(printf, 2
 // lives.  The calls of one owner share its buffers and therefore run in the
 // order of one stream.
 struct WorkBufs {
-    enum Slot { TAPE, GACC, PART, PARAMS, SPOT_PART, SPOT_CS, DESCEND, EXT_KEYS, SAVE_HIST, SAVE_LPOS, SAVE_TILES,
+    enum Slot { TAPE, PARAMS, SPOT_PART, SPOT_CS, DESCEND, EXT_KEYS, SAVE_HIST, SAVE_LPOS, SAVE_TILES,
                 SAVE_GPOS, TRACE_PART, N_SLOTS };
     void* p[N_SLOTS] = {};
     size_t have[N_SLOTS] = {};
@@ -84,14 +84,10 @@ struct BatchView {
 int rt_batch_view(const rt_hip_batch* b, BatchView* v);
 WorkBufs* rt_batch_work(const rt_hip_batch* b);
 
-// The per-wavelength table of a scheme or batch (its spline-valued functions
-// at the grid wavelengths of a beam): the number of grid wavelengths it
+// The per-wavelength table of a scheme or batch: the number of grid wavelengths it
 // serves for this beam description, 0 when it does not (random wavelengths,
 // no spline-valued function, tables disabled); and its filling on `stream`
 // (*tab: the device table, column q at q * nk).
-uint64_t rt_scheme_ltab_nk(const rt_hip_scheme* s, const double* beam_desc);
-int rt_scheme_ltab_fill(const rt_hip_scheme* s, const double* beam_desc, uint64_t nk, hipStream_t stream,
-                        const double** tab);
 // The derived per-wavelength table of a scheme (mu, grating term, flux
 // weight; the layout of rt_jit_dtab_layout), likewise; kept while the grid
 // and the stream stay those of its last fill.

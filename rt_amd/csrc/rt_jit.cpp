@@ -36,6 +36,7 @@ struct Entry {
     hipFunction_t fn = nullptr;
     bool failed = false;
     std::string log;
+    int tape_rows = 0;               // adjoint kernels: the tape's rows in memory
 };
 std::map<std::string, Entry> g_cache;
 
@@ -312,11 +313,6 @@ static AdjTape adjoint_tape(const std::vector<std::string>& types) {
     return t;
 }
 
-int rt_jit_adjoint_tape_rows(const std::string& sig, int lds_rows) {
-    const AdjTape t = adjoint_tape(sig_types(sig));
-    return std::max(1, t.total - std::min(lds_rows, t.state));
-}
-
 static std::string generate_adjoint_source(const std::string& sig, int beam_type, const std::vector<int>& rows,
                                            int n_surf, int block, int waves = 0, bool batch = false,
                                            bool ltab = false, int lds_rows = 0) {
@@ -557,7 +553,8 @@ hipFunction_t rt_jit_kernel(const std::string& sig, int beam_mode, int variant, 
 }
 
 hipFunction_t rt_jit_adjoint_kernel(const std::string& sig, int beam_type, const std::vector<int>& rows, int n_surf,
-                                    int block, int waves, int device, bool batch, bool ltab, int lds_rows) {
+                                    int block, int waves, int device, bool batch, bool ltab, int lds_rows,
+                                    int* tape_rows) {
     std::ostringstream key;
     key << device << "|adjoint|" << (batch ? "batch|" : "") << (ltab ? "ltab|" : "") << beam_type << "|" << block
         << "|" << waves << "|" << lds_rows << "|";
@@ -566,8 +563,11 @@ hipFunction_t rt_jit_adjoint_kernel(const std::string& sig, int beam_type, const
     key << "|" << sig;
     std::lock_guard<std::mutex> lk(g_mu);
     Entry& e = g_cache[key.str()];
-    if (e.fn) return e.fn;
     if (e.failed) return nullptr;
+    if (e.fn) {
+        *tape_rows = e.tape_rows;
+        return e.fn;
+    }
     if (!compile(generate_adjoint_source(sig, beam_type, rows, n_surf, block, waves, batch, ltab, lds_rows), e,
                  "rt_adjoint_jit")) {
         e.failed = true;
@@ -575,6 +575,8 @@ hipFunction_t rt_jit_adjoint_kernel(const std::string& sig, int beam_type, const
                 e.log.c_str());
         return nullptr;
     }
+    const AdjTape tape = adjoint_tape(sig_types(sig));
+    *tape_rows = e.tape_rows = std::max(1, tape.total - std::min(lds_rows, tape.state));
     return e.fn;
 }
 

@@ -51,11 +51,8 @@ hipFunction_t rt_jit_kernel(const std::string& signature, int beam_mode, int var
 // or -1.  Compiled on first use and cached; nullptr on failure (the caller
 // launches the generic adjoint kernel).
 // lds_rows: tape rows a lane keeps in LDS (8 bytes x block of dynamic LDS
-// each; the kernel then stages no pool).
+// each; the kernel then stages no pool); *tape_rows: its rows in memory (the
+// generic kernel uses n_surf x kTape).
 hipFunction_t rt_jit_adjoint_kernel(const std::string& signature, int beam_type, const std::vector<int>& rows,
                                     int n_surf, int block, int waves, int device, bool batch,
-                                    bool ltab = false, int lds_rows = 0);
-
-// Tape rows per lane in memory of the generated adjoint kernels of a
-// signature; the generic adjoint kernel uses n_surf x kTape.
-int rt_jit_adjoint_tape_rows(const std::string& signature, int lds_rows);
+                                    bool ltab, int lds_rows, int* tape_rows);

@@ -499,12 +499,6 @@ struct Dtab {
     bool always = false;             // a launch was captured: fill every time
     double key[5] = {0, 0, 0, 0, 0};
     hipStream_t stream = nullptr;    // stream of the last fill
-    void release() {
-        (void)hipFree(tab_dev);
-        tab_dev = nullptr;
-        n_cols = 0;
-        valid = false;
-    }
 };
 
 struct rt_hip_scheme {
@@ -531,7 +525,7 @@ struct rt_hip_scheme {
     // surface unroll depth: 1, the whole chain unrolled (the generated
     // kernel); 0, a runtime loop over the records (the generic kernel)
     int unroll = 1;
-    Ltab lt;
+    void* arena = nullptr;           // the allocation of table_dev, pool_dev, stat_copies and dt.tab_dev
     // kStatCopies x RT_STATS_LEN counters the trace kernels add to, folded into
     // the caller's statistics after each trace (and cleared by the fold)
     unsigned long long* stat_copies = nullptr;
@@ -800,14 +794,11 @@ uint64_t grid_nk(const double* beam) {
 
 uint64_t ltab_nk(const Ltab& t, const double* beam) { return t.ok ? grid_nk(beam) : 0; }
 
-// the derived table's columns for the signature; its buffer on first use
-int dtab_setup(Dtab& t, const std::string& sig) {
+// the derived table's columns for the signature
+void dtab_layout(Dtab& t, const std::string& sig) {
     std::vector<int> base, surf, role;
     rt_jit_dtab_layout(sig, base, surf, role);
     t.n_cols = (int)surf.size();
-    if (t.n_cols > 0 && !t.tab_dev)
-        HIP_TRY(hipMalloc(&t.tab_dev, (size_t)t.n_cols * kLtabMax * sizeof(double)), RT_ERR_BAD_ALLOC);
-    return RT_OK;
 }
 
 uint64_t dtab_nk(const Dtab& t, const double* beam) { return t.n_cols > 0 ? grid_nk(beam) : 0; }
@@ -874,35 +865,31 @@ extern "C" int rt_hip_scheme_create(const double* surf_table, int n_surf, const 
     s->table.assign(surf_table, surf_table + (size_t)n_surf * RT_SURF_STRIDE);
     if (pool_len) s->pool.assign(spline_pool, spline_pool + pool_len);
     build_device_tables(s);
-    s->table_dev = nullptr;
-    s->pool_dev = nullptr;
-    size_t tb = s->dtable.size() * sizeof(double);
-    size_t pb = (s->dpool.empty() ? 1 : s->dpool.size()) * sizeof(double);
-    if (hipMalloc(&s->table_dev, tb) != hipSuccess || hipMalloc(&s->pool_dev, pb) != hipSuccess) {
-        (void)hipFree(s->table_dev);
-        (void)hipFree(s->pool_dev);
+    // one allocation and one upload for all: a scheme made and destroyed, as each
+    // evaluation of a loss does, 68 -> 41 us
+    dtab_layout(s->dt, s->signature);
+    const size_t stats = (size_t)rt::kStatCopies * RT_STATS_LEN * sizeof(unsigned long long);
+    const size_t tb = (s->dtable.size() * sizeof(double) + 255) / 256 * 256;
+    const size_t pb = ((s->dpool.empty() ? 1 : s->dpool.size()) * sizeof(double) + 255) / 256 * 256;
+    const size_t dt = (size_t)s->dt.n_cols * kLtabMax * sizeof(double);
+    char* dev = nullptr;
+    if (hipMalloc(&dev, tb + pb + stats + dt) != hipSuccess) {
         delete s;
         return set_error(RT_ERR_BAD_ALLOC, "hipMalloc of scheme tables failed");
     }
-    if (hipMemcpy(s->table_dev, s->dtable.data(), tb, hipMemcpyHostToDevice) != hipSuccess ||
-        (!s->dpool.empty() && hipMemcpy(s->pool_dev, s->dpool.data(), s->dpool.size() * sizeof(double),
-                                        hipMemcpyHostToDevice) != hipSuccess)) {
-        (void)hipFree(s->table_dev);
-        (void)hipFree(s->pool_dev);
+    s->arena = dev;
+    s->table_dev = (double*)dev;
+    s->pool_dev = (double*)(dev + tb);
+    s->stat_copies = (unsigned long long*)(dev + tb + pb);
+    s->dt.tab_dev = dt ? (double*)(dev + tb + pb + stats) : nullptr;
+    std::vector<double> up((tb + pb) / sizeof(double), 0.0);
+    std::copy(s->dtable.begin(), s->dtable.end(), up.begin());
+    std::copy(s->dpool.begin(), s->dpool.end(), up.begin() + tb / sizeof(double));
+    if (hipMemset(s->stat_copies, 0, stats) != hipSuccess ||
+        hipMemcpy(dev, up.data(), tb + pb, hipMemcpyHostToDevice) != hipSuccess) {
+        (void)hipFree(dev);
         delete s;
         return set_error(RT_ERR_FAILED, "upload of scheme tables failed");
-    }
-    rc = ltab_setup(s->lt, s->signature, s->dtable.data(), 1, n_surf);
-    if (rc == RT_OK) rc = dtab_setup(s->dt, s->signature);
-    if (rc == RT_OK) rc = stat_copies_alloc(&s->stat_copies);
-    if (rc != RT_OK) {
-        (void)hipFree(s->stat_copies);
-        s->lt.release();
-        s->dt.release();
-        (void)hipFree(s->table_dev);
-        (void)hipFree(s->pool_dev);
-        delete s;
-        return rc;
     }
     *out = s;
     return RT_OK;
@@ -927,11 +914,7 @@ extern "C" int rt_hip_jit_check(const double* surf_table, int n_surf, const doub
 extern "C" int rt_hip_scheme_destroy(rt_hip_scheme* s) {
     if (!s) return RT_OK;
     s->work.release();
-    (void)hipFree(s->stat_copies);
-    s->lt.release();
-    s->dt.release();
-    (void)hipFree(s->table_dev);
-    (void)hipFree(s->pool_dev);
+    (void)hipFree(s->arena);
     delete s;
     return RT_OK;
 }
@@ -1879,17 +1862,6 @@ int rt_batch_view(const rt_hip_batch* b, BatchView* v) {
 }
 
 const std::string& rt_scheme_signature(const rt_hip_scheme* s) { return s->signature; }
-
-uint64_t rt_scheme_ltab_nk(const rt_hip_scheme* s, const double* beam_desc) { return ltab_nk(s->lt, beam_desc); }
-
-int rt_scheme_ltab_fill(const rt_hip_scheme* s, const double* beam_desc, uint64_t nk, hipStream_t stream,
-                        const double** tab) {
-    TraceArgs a;
-    memset(&a, 0, sizeof a);
-    memcpy(a.beam.v, beam_desc, sizeof a.beam.v);
-    *tab = s->lt.tab_dev;
-    return ltab_fill(s->lt, a, s->pool_dev, nk, stream);
-}
 
 uint64_t rt_scheme_dtab_nk(const rt_hip_scheme* s, const double* beam_desc) { return dtab_nk(s->dt, beam_desc); }
 

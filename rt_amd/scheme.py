@@ -263,19 +263,18 @@ def pack_surfaces(surfaces: Sequence[Surface]) -> Tuple[np.ndarray, np.ndarray]:
     if len(surfaces) > RT_MAX_SURF:
         raise ValueError("too many surfaces")
     table = np.zeros((len(surfaces), SURF_STRIDE))
-    pool: List[float] = []
+    pool: List[np.ndarray] = []
     offsets = {}
+    size = 0
 
     def ref(fn: FnRef) -> Tuple[float, float]:
+        nonlocal size
         if isinstance(fn, Spline):
             key = id(fn)
             if key not in offsets:
-                offsets[key] = len(pool)
-                k = len(fn.x)
-                pool.append(float(k))
-                pool.extend(fn.x.tolist())
-                pool.extend(fn.y.tolist())
-                pool.extend(fn.y2.tolist())
+                offsets[key] = size
+                pool.extend(([float(len(fn.x))], fn.x, fn.y, fn.y2))
+                size += 1 + len(fn.x) + len(fn.y) + len(fn.y2)
             return float(RT_FN_SPLINE), float(offsets[key])
         return float(RT_FN_CONST), float(fn)
 
@@ -312,9 +311,8 @@ def pack_surfaces(surfaces: Sequence[Surface]) -> Tuple[np.ndarray, np.ndarray]:
             r[S_CCD_YSIZE] = c.get("ysize", c["ydim"] * c["ypix"])
             r[S_QEKIND], r[S_QEVAL] = ref(s.qe)
             r[S_SPKIND], r[S_SPVAL] = ref(s.spectrum)
-    if not pool:
-        pool = [0.0]
-    return table.reshape(-1).copy(), np.asarray(pool, dtype=np.float64)
+    flat = np.concatenate(pool) if pool else [0.0]
+    return table.reshape(-1), np.asarray(flat, dtype=np.float64)
 
 
 # ---- geometry helper: aim the next surface along a chief ray ----------------
