@@ -953,11 +953,22 @@ namespace {
 // loads and on splines in LDS: 1e6 echelle rays 121 -> 112 us) and, where both
 // frames take an atomic of every ray and bound the trace, workgroups of 512
 // lanes from 2^20 rays on (1e7 echelle rays 926 -> 892 us; with fewer rays, or
-// one frame or none, 256 lanes are as fast or faster).
+// one frame or none, 256 lanes are as fast or faster); and 1024 lanes and 8
+// waves per SIMD for recording traces with extents from 2^18 rays on, where
+// every workgroup has to meet the extremes before its rays lie inside them
+// (2^18 echelle rays 53 -> 47 us, 2^20 161 -> 123, 2^22 485 -> 401; 2^17 39 ->
+// 46, so not there).
 void trace_shape(const rt_hip_scheme* sch, bool gen, const TraceArgs& a, int rec, int& block, int& waves) {
     block = sch->block;
     waves = sch->waves;
-    if (sch->launch_given || rec) return;
+    if (sch->launch_given) return;
+    if (rec) {
+        if ((rec & rt::kRecExt) && a.n >= (1u << 18)) {
+            block = 1024;
+            waves = 8;
+        }
+        return;
+    }
     if (!gen) waves = 8;
     const bool frames = (a.flags & RT_TRACE_HIST) && a.hist && (a.flags & RT_TRACE_FLUX) && a.flux;
     if (gen && frames && a.n >= (1u << 20)) block = 512;

@@ -141,7 +141,7 @@ def test_rearrange_order_and_counts(hip, n, offset, lost):
 
 # one ray, a partial workgroup, and more rays than the resident workgroups take
 # in one round (so that each meets rays inside and outside its bounds)
-@pytest.mark.parametrize("n", [1, 300, 700003])
+@pytest.mark.parametrize("n", [1, 300, (1 << 18) - 1, 1 << 18, 700003])
 def test_recorded_extents_equal_dumped_states(hip, n):
     print(f"[extents] n={n}", flush=True)
     from rt_amd import scheme as S, schemes
