@@ -354,7 +354,10 @@ int rt_hip_set_ltab(int mode);
    powers of two), the minimum number of waves per SIMD the compiler must fit
    its registers to (0: its own choice), and persistent workgroups per CU as a
    multiple of those that are resident at once.  Default 256, 7, 16 (for
-   schemes and batches).  No counterpart in the reference (its launches are
+   schemes and batches; a scheme whose launch is never set takes 8 waves for
+   rays given by the caller, 512 lanes for large traces with both frames, and
+   1024 lanes and 8 waves for large recording traces with extents).  No
+   counterpart in the reference (its launches are
    fixed per kernel). */
 int rt_hip_scheme_set_launch(rt_hip_scheme *scheme, int block, int waves, int grid_mult);
 int rt_hip_scheme_get_launch(const rt_hip_scheme *scheme, int *block, int *waves, int *grid_mult);
