@@ -982,6 +982,14 @@ unsigned ext_grid(uint64_t tiles, uint64_t resident) {
     return (unsigned)((tiles + rounds - 1) / rounds);
 }
 
+template <int MODE>
+auto generic_kernel(int beam_mode) {
+    return beam_mode == RT_BEAM_PARALLEL ? rt_trace_kernel<RT_BEAM_PARALLEL, MODE>
+           : beam_mode == RT_BEAM_CONIC  ? rt_trace_kernel<RT_BEAM_CONIC, MODE>
+           : beam_mode == RT_BEAM_GAUSS  ? rt_trace_kernel<RT_BEAM_GAUSS, MODE>
+                                         : rt_trace_kernel<kLoad, MODE>;
+}
+
 // rt_hip_trace and rt_hip_trace_record: rec is the recording mode (rt::kRecLoss
 // | rt::kRecExt or 0), loss / extents its outputs
 int trace_launch(const rt_hip_scheme* sch, const double* beam_desc, uint64_t seed, size_t ray_begin, size_t n_rays,
@@ -1090,18 +1098,12 @@ int trace_launch(const rt_hip_scheme* sch, const double* beam_desc, uint64_t see
             rc = ext_rows(cap);
             if (rc != RT_OK) return rc;
         }
-        constexpr int R = rt::kRecLoss | rt::kRecExt, SP = rt::kRecSpots;
-        auto kern = rec == 0 ? (beam_mode == RT_BEAM_PARALLEL ? rt_trace_kernel<RT_BEAM_PARALLEL>
-                                : beam_mode == RT_BEAM_CONIC  ? rt_trace_kernel<RT_BEAM_CONIC>
-                                : beam_mode == RT_BEAM_GAUSS  ? rt_trace_kernel<RT_BEAM_GAUSS>
-                                                              : rt_trace_kernel<kLoad>)
-                  : rec == SP ? (beam_mode == RT_BEAM_PARALLEL ? rt_trace_kernel<RT_BEAM_PARALLEL, SP>
-                                 : beam_mode == RT_BEAM_CONIC  ? rt_trace_kernel<RT_BEAM_CONIC, SP>
-                                                               : rt_trace_kernel<RT_BEAM_GAUSS, SP>)
-                             : (beam_mode == RT_BEAM_PARALLEL ? rt_trace_kernel<RT_BEAM_PARALLEL, R>
-                                : beam_mode == RT_BEAM_CONIC  ? rt_trace_kernel<RT_BEAM_CONIC, R>
-                                : beam_mode == RT_BEAM_GAUSS  ? rt_trace_kernel<RT_BEAM_GAUSS, R>
-                                                              : rt_trace_kernel<kLoad, R>);
+        // (a kernel that records extents writes its keys: the one without them
+        // where the caller wants none)
+        auto kern = rec == 0                                ? generic_kernel<0>(beam_mode)
+                    : rec == rt::kRecSpots                  ? generic_kernel<rt::kRecSpots>(beam_mode)
+                    : rec == (rt::kRecLoss | rt::kRecExt)   ? generic_kernel<rt::kRecLoss | rt::kRecExt>(beam_mode)
+                                                            : generic_kernel<rt::kRecLoss>(beam_mode);
         stats_target(a, sch->stat_copies, stats, grid);
         hipLaunchKernelGGL(kern, dim3(grid), dim3(kBlock), lds, st, a);
         g_last_kernel = "generic";

@@ -166,6 +166,36 @@ def test_recorded_extents_equal_dumped_states(hip, n):
     ds.close()
 
 
+# extents are optional: without them the generic kernel records the same codes
+# and rays as with them, and as the generated kernel
+@pytest.mark.parametrize("n", [1, 700])
+def test_recording_without_extents(hip, n):
+    from rt_amd import schemes
+    sc = schemes.echelle_fixed_order(n, 1)
+    out = []
+    for jit, want in ((False, True), (False, False), (True, False)):
+        print(f"[recording] n={n} generated={jit} extents={want}", flush=True)
+        prev = hip.set_jit(jit)
+        try:
+            ds = hip.DeviceScheme(sc)
+            rays = torch.empty((7, n), dtype=torch.float64, device="cuda")
+            flag, loss = (torch.empty(n, dtype=d, device="cuda") for d in (torch.int8, torch.uint8))
+            ext = torch.zeros((sc.n_surf, hip.EXT_PER_SURF), dtype=torch.float64, device="cuda") if want else None
+            ds.trace_record(rays, flag, loss, seed=6, extents=ext)
+            out.append((rays.cpu().numpy(), flag.cpu().numpy(), loss.cpu().numpy()))
+            ds.close()
+        finally:
+            hip.set_jit(prev)
+    for got in out[1:]:
+        assert np.array_equal(got[1], out[0][1]) and np.array_equal(got[2], out[0][2])
+    assert np.array_equal(out[1][0], out[0][0])
+    # two kernels from the same stage code: 1e-12 of the scheme's length, of a
+    # unit direction and of the wavelength
+    L = max(1.0, max(abs(d) for q in sc.surfaces for d in q.distance))
+    scale = np.array([L, L, L, 1.0, 1.0, 1.0, 1.0])[:, None]
+    assert np.all(np.abs(out[2][0] - out[0][0]) <= 1e-12 * scale)
+
+
 def every_surface_kind():
     """a lens, a rotated auxiliary frame, a rotated stop, an aspheric and a
     toric lens, a plane lens face, both kinds of grating, a spherical and a
