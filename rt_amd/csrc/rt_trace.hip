@@ -948,6 +948,10 @@ static void beam_uniforms(TraceArgs& a) {
 }
 
 namespace {
+// recording traces with extents: rays from which their launch is the large one,
+// and the workgroups of the default launch that the rays below it take at most
+constexpr uint64_t kExtRays = 1u << 18, kExtTiles = kExtRays / kBlock;
+
 // The launch of a trace of a scheme whose launch nobody has set: the defaults,
 // but 8 waves per SIMD for rays given by the caller (their kernel waits on its
 // loads and on splines in LDS: 1e6 echelle rays 121 -> 112 us) and, where both
@@ -963,7 +967,7 @@ void trace_shape(const rt_hip_scheme* sch, bool gen, const TraceArgs& a, int rec
     waves = sch->waves;
     if (sch->launch_given) return;
     if (rec) {
-        if ((rec & rt::kRecExt) && a.n >= (1u << 18)) {
+        if ((rec & rt::kRecExt) && a.n >= kExtRays) {
             block = 1024;
             waves = 8;
         }
@@ -1042,12 +1046,24 @@ int trace_launch(const rt_hip_scheme* sch, const double* beam_desc, uint64_t see
     unsigned grid = 0;
     int block, waves;
     trace_shape(sch, gen, a, rec, block, waves);
-    // the rows of extents keys of as many workgroups as this launch can have
-    auto ext_rows = [&](uint64_t most) {
-        const int r = sch->work.ensure(WorkBufs::EXT_KEYS,
-                                       (size_t)sch->n_surf * rt::kExtPerSurf * most * sizeof(unsigned long long));
-        if (r == RT_OK) a.ext = sch->work.get<unsigned long long>(WorkBufs::EXT_KEYS);
-        return r;
+    // The workgroups of a recording trace with extents, and their rows of keys:
+    // at least the rows that any size of the default launches takes, so that a
+    // later call of another size finds its memory there, also while a graph is
+    // captured; a capture of a launch that could use more (smaller workgroups,
+    // set since) has as many workgroups as there are rows.
+    auto ext_launch = [&](uint64_t tiles, uint64_t resident) -> int {
+        const size_t row = (size_t)sch->n_surf * rt::kExtPerSurf * sizeof(unsigned long long);
+        const size_t bytes = row * std::max<uint64_t>(kExtTiles, std::min(tiles, resident));
+        const size_t& have = sch->work.have[WorkBufs::EXT_KEYS];
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        if (have > 0 && have < bytes) HIP_TRY(hipStreamIsCapturing(st, &cs), RT_ERR_FAILED);
+        if (cs == hipStreamCaptureStatusNone) {
+            const int r = sch->work.ensure(WorkBufs::EXT_KEYS, bytes);
+            if (r != RT_OK) return r;
+        }
+        a.ext = sch->work.get<unsigned long long>(WorkBufs::EXT_KEYS);
+        grid = ext_grid(tiles, std::min<uint64_t>(resident, have / row));
+        return RT_OK;
     };
     hipFunction_t fn = nullptr;
     if (rt_jit_enabled() && sch->unroll)
@@ -1074,11 +1090,7 @@ int trace_launch(const rt_hip_scheme* sch, const double* beam_desc, uint64_t see
         uint64_t want = (n_rays + block - 1) / block;
         uint64_t cap = (uint64_t)cus * resident * sch->grid_mult;
         grid = (unsigned)(want < cap ? want : cap);
-        if (extents) {
-            grid = ext_grid(want, (uint64_t)cus * resident);
-            rc = ext_rows((uint64_t)cus * resident);
-            if (rc != RT_OK) return rc;
-        }
+        if (extents && (rc = ext_launch(want, (uint64_t)cus * resident)) != RT_OK) return rc;
         stats_target(a, sch->stat_copies, stats, grid);
         void* params[] = {&a};
         HIP_TRY(hipModuleLaunchKernel(fn, grid, 1, 1, block, 1, 1, (unsigned)lds, st, params, nullptr),
@@ -1093,11 +1105,7 @@ int trace_launch(const rt_hip_scheme* sch, const double* beam_desc, uint64_t see
         uint64_t want = (n_rays + kBlock - 1) / kBlock;
         uint64_t cap = (uint64_t)cus * 8;      // persistent grid: 8 blocks (32 waves) per CU
         grid = (unsigned)(want < cap ? want : cap);
-        if (extents) {
-            grid = ext_grid(want, cap);
-            rc = ext_rows(cap);
-            if (rc != RT_OK) return rc;
-        }
+        if (extents && (rc = ext_launch(want, cap)) != RT_OK) return rc;
         // (a kernel that records extents writes its keys: the one without them
         // where the caller wants none)
         auto kern = rec == 0                                ? generic_kernel<0>(beam_mode)

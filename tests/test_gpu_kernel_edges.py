@@ -196,6 +196,50 @@ def test_recording_without_extents(hip, n):
     assert np.all(np.abs(out[2][0] - out[0][0]) <= 1e-12 * scale)
 
 
+# recordings of another size than the one before them, captured in a graph:
+# nothing is allocated then, whatever launch the size takes, nor for a launch
+# of smaller workgroups set in between
+@pytest.mark.parametrize("first,then,block", [(1 << 18, 5000, None), (5000, 1 << 18, None), (1 << 18, 1 << 18, 64)])
+def test_recording_captured_after_another_size(hip, first, then, block):
+    print(f"[captured recording] {first} then {then}, {block}", flush=True)
+    from rt_amd import schemes
+    sc = schemes.echelle_fixed_order(1 << 18, 1)
+    m = max(first, then)
+    rays = torch.empty((7, m), dtype=torch.float64, device="cuda")
+    flag, loss = (torch.empty(m, dtype=d, device="cuda") for d in (torch.int8, torch.uint8))
+    ext = torch.zeros((sc.n_surf, hip.EXT_PER_SURF), dtype=torch.float64, device="cuda")
+    stream = torch.cuda.Stream()
+
+    def record(ds, n):
+        ds.trace_record(rays, flag, loss, seed=4, n=n, extents=ext, stream=stream.cuda_stream)
+    ds = hip.DeviceScheme(sc)
+    with torch.cuda.stream(stream):
+        record(ds, then)                                   # the kernels of both sizes are compiled
+        want = ext.clone()
+        record(ds, first)
+    stream.synchronize()
+    ds.close()
+    ds = hip.DeviceScheme(sc)                              # a scheme without working memory yet
+    with torch.cuda.stream(stream):
+        record(ds, first)
+    stream.synchronize()
+    if block:
+        ds.set_launch(block, 8, 16)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=stream, capture_error_mode="thread_local"):
+        record(ds, then)
+    for k in range(3):
+        ext.zero_()
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(ext, want), k
+        with torch.cuda.stream(stream):
+            record(ds, first)
+        torch.cuda.synchronize()
+    ds.close()
+
+
 def every_surface_kind():
     """a lens, a rotated auxiliary frame, a rotated stop, an aspheric and a
     toric lens, a plane lens face, both kinds of grating, a spherical and a
