@@ -68,8 +68,14 @@ __device__ void block_add(unsigned long long* dst, unsigned long long v) {
 // so the stages that count add per workgroup, at most kCountBlocks of them (a
 // mask that loses rays in every wave: 113 -> 11 us at 1e6 rays with an add per
 // wave before; a Newton intersection 53 -> 20 us with one per 256 rays).
+// Workgroups of 1024 lanes keep the memory busy with that few (the echelle's
+// 12 surfaces stage by stage at 1e6 rays 777 us, with 256 lanes 784, at 2e6
+// 1,408 and 1,495); up to kCountSmall rays they leave CUs without one, or with
+// one round of work where others have two, and 256 lanes are faster (3e5 rays
+// 374 against 464 us, 6e5 526 against 575).
 constexpr int kCountThreads = 1024;
 constexpr unsigned kCountBlocks = 512;
+constexpr size_t kCountSmall = 3u << 18;
 
 // frame change: which coordinates move (the same for every ray)
 struct Touch {
@@ -311,9 +317,11 @@ unsigned grid_for(size_t n) {
     return (unsigned)(want < cap ? (want ? want : 1) : cap);
 }
 
-// workgroups of kCountThreads lanes of a counting kernel
+// lanes and workgroups of a counting kernel
+unsigned count_threads(size_t n) { return n < kCountSmall ? kThreads : kCountThreads; }
+
 unsigned count_grid(size_t n) {
-    const uint64_t want = (n + kCountThreads - 1) / kCountThreads;
+    const uint64_t want = (n + count_threads(n) - 1) / count_threads(n);
     return (unsigned)(want < kCountBlocks ? (want ? want : 1) : kCountBlocks);
 }
 
@@ -337,7 +345,7 @@ int launch_stage(const double* rec, size_t n, int op, double* X, double* Y, doub
                 : op == OP_REFLECT   ? rt_reflect_kernel
                 : op == OP_REFRACT   ? rt_count_stage_kernel<OP_REFRACT>
                                      : rt_count_stage_kernel<OP_DIFFRACT>;
-    hipLaunchKernelGGL(kern, dim3(count ? count_grid(n) : grid_for(n)), dim3(count ? kCountThreads : kThreads), 0,
+    hipLaunchKernelGGL(kern, dim3(count ? count_grid(n) : grid_for(n)), dim3(count ? count_threads(n) : kThreads), 0,
                        (hipStream_t)stream, a);
     HIP_TRY(hipGetLastError(), RT_ERR_FAILED);
     return RT_OK;
@@ -491,7 +499,7 @@ extern "C" int rt_hip_ccd_accumulate(size_t n, const unsigned* ccdX, const unsig
     a.n = n; a.xdim = (uint32_t)xdim; a.ydim = (uint32_t)ydim;
     a.ccdX = (unsigned*)ccdX; a.ccdY = (unsigned*)ccdY; a.w = w; a.image = image; a.hist = hist;
     a.offchip = offchip;
-    hipLaunchKernelGGL(rt_ccd_accumulate_kernel, dim3(count_grid(n)), dim3(kCountThreads), 0, (hipStream_t)stream, a);
+    hipLaunchKernelGGL(rt_ccd_accumulate_kernel, dim3(count_grid(n)), dim3(count_threads(n)), 0, (hipStream_t)stream, a);
     HIP_TRY(hipGetLastError(), RT_ERR_FAILED);
     return RT_OK;
 }

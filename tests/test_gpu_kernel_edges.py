@@ -45,9 +45,10 @@ def test_group_spots_at_chunk_edges(hip, n, G):
     assert np.all(np.abs(got[:, 3:6] - want[:, 3:6]) <= 1e-10 * np.abs(want[:, 3:6]) + 1e-28)
 
 
-# one lane, one wave, a workgroup of the counting stages and its neighbours,
-# more rays than their largest grid holds at once
-@pytest.mark.parametrize("n", [1, 64, 1023, 1024, 1025, 512 * 1024 + 1])
+# one lane, one wave, the counting stages' workgroups of 256 lanes and of 1024
+# (from 3 * 2^18 rays on), more rays than their largest grids hold at once
+@pytest.mark.parametrize("n", [1, 64, 255, 257, 1023, 1024, 1025, 512 * 256 + 1, 512 * 1024 + 1, (3 << 18) - 1,
+                               3 << 18, (3 << 18) + 1])
 def test_mask_counts_and_flags(hip, n):
     print(f"[mask] n={n}", flush=True)
 
