@@ -1732,18 +1732,7 @@ __device__ __forceinline__ void trace_body(const TraceArgs& a, Surfaces surfaces
             // the ray pointers are read from the argument segment where they are
             // used, not held in SGPRs across the surface chain
             const cargs ka = kernel_args();
-            if (ka->X && (c.do_hist || c.do_flux)) {
-                // rows that stream past the frames: without a place in the
-                // caches they leave the frames theirs (echelle of 1e7 rays,
-                // both frames and the rays: 892 -> 880 us)
-                __builtin_nontemporal_store(r.X, &ka->X[i]);
-                __builtin_nontemporal_store(r.Y, &ka->Y[i]);
-                __builtin_nontemporal_store(r.Z, &ka->Z[i]);
-                __builtin_nontemporal_store(r.cX, &ka->cX[i]);
-                __builtin_nontemporal_store(r.cY, &ka->cY[i]);
-                __builtin_nontemporal_store(r.cZ, &ka->cZ[i]);
-                __builtin_nontemporal_store(r.lam, &ka->L[i]);
-            } else if (ka->X) {
+            if (ka->X) {
                 ka->X[i] = r.X; ka->Y[i] = r.Y; ka->Z[i] = r.Z;
                 ka->cX[i] = r.cX; ka->cY[i] = r.cY; ka->cZ[i] = r.cZ;
                 ka->L[i] = r.lam;
