@@ -353,12 +353,16 @@ int rt_hip_set_ltab(int mode);
 /* Launch of a scheme's generated kernel: lanes per workgroup (64..1024,
    powers of two), the minimum number of waves per SIMD the compiler must fit
    its registers to (0: its own choice), and persistent workgroups per CU as a
-   multiple of those that are resident at once.  Default 256, 7, 16 (for
-   schemes and batches; a scheme whose launch is never set takes 8 waves for
+   multiple of those that are resident at once (recording traces with extents:
+   as many as are resident, whatever the multiple).  Default 256, 7, 16 (for
+   schemes and batches; a scheme whose launch nobody set takes 8 waves for
    rays given by the caller, 512 lanes for large traces with both frames, and
-   1024 lanes and 8 waves for large recording traces with extents).  No
-   counterpart in the reference (its launches are
-   fixed per kernel). */
+   1024 lanes and 8 waves for large recording traces with extents).  A launch
+   that was set holds for every trace of the scheme, one from the autotuner
+   for traces like those it timed.  rt_hip_scheme_get_launch returns the launch
+   that was set or tuned, the default for a scheme without one: not what those
+   rules make of it for a particular trace.  No counterpart in the reference
+   (its launches are fixed per kernel). */
 int rt_hip_scheme_set_launch(rt_hip_scheme *scheme, int block, int waves, int grid_mult);
 int rt_hip_scheme_get_launch(const rt_hip_scheme *scheme, int *block, int *waves, int *grid_mult);
 
@@ -373,14 +377,17 @@ int rt_hip_scheme_get_unroll(const rt_hip_scheme *scheme, int *full);
 /* Autotuner: traces n_sample rays of the beam (generated from seed, seed + 1,
    ... for successive launches, with `flags`) under each candidate launch
    (block 128/256, waves 0/5/6/7/8, grid multiple 1/2/4/8/16 of the fully
-   unrolled generated kernel, and the runtime surface loop of the generic
-   kernel; those spilling more than 64 bytes per lane to scratch are set
+   unrolled generated kernel, for large samples into both frames block 512
+   too, and the runtime surface loop of the generic kernel; those spilling more than 64 bytes per lane to scratch are set
    aside when others exist) in
    3 interleaved rounds of 3 back-to-back launches, re-times the four fastest
    in 5 rounds of 20 (a sustained load runs at a lower clock than isolated
    launches, by an amount that depends on the launch), keeps the one with the
    lowest median (within 0.5%, the one with less scratch memory per lane) in
-   the scheme and returns that median (per launch) in *best_ms.
+   the scheme and returns that median (per launch) in *best_ms.  The launch
+   kept is that of the scheme's generated traces that record nothing and form
+   both frames, or not both, as `flags` says; other traces keep the launches
+   of a scheme without one (and no longer take one set before).
    RT_HIP_AUTOTUNE_LOG=1 prints every candidate's times on stderr.  Allocates
    its sample buffers; call it once after rt_hip_scheme_create, outside any
    timed or captured region. */

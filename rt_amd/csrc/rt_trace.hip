@@ -501,6 +501,8 @@ struct Dtab {
     hipStream_t stream = nullptr;    // stream of the last fill
 };
 
+constexpr int kDefaultWaves = 7, kDefaultGridMult = 16;
+
 struct rt_hip_scheme {
     int device;
     std::string signature;           // structural key of the generated kernels
@@ -519,9 +521,12 @@ struct rt_hip_scheme {
     // the batched trace over 1024 instances of uneven size, 21.3 ms against
     // 23.7-24.0 ms at a grid multiple of 2)
     int block = rt::kBlock;          // lanes per workgroup
-    int waves = 7;                   // minimum waves per SIMD asked of the compiler (0: its choice)
-    int grid_mult = 16;              // persistent workgroups per CU = grid_mult x resident ones
-    bool launch_given = false;       // set by the caller or the autotuner: taken as it is
+    int waves = kDefaultWaves;       // minimum waves per SIMD asked of the compiler (0: its choice)
+    int grid_mult = kDefaultGridMult;    // persistent workgroups per CU = grid_mult x resident ones
+    // who set them: nobody (launch_shape's rules hold), the autotuner (taken for
+    // the traces it timed) or the caller (taken for every trace)
+    enum { BY_RULE, BY_TUNER, BY_CALLER } launch_by = BY_RULE;
+    bool tuned_frames = false;       // the autotuner's traces formed both frames
     // surface unroll depth: 1, the whole chain unrolled (the generated
     // kernel); 0, a runtime loop over the records (the generic kernel)
     int unroll = 1;
@@ -951,31 +956,43 @@ namespace {
 // recording traces with extents: rays from which their launch is the large one,
 // and the workgroups of the default launch that the rays below it take at most
 constexpr uint64_t kExtRays = 1u << 18, kExtTiles = kExtRays / kBlock;
+// generated rays into both frames from which a workgroup has 512 lanes
+constexpr uint64_t kFrameRays = 1u << 20;
 
-// The launch of a trace of a scheme whose launch nobody has set: the defaults,
-// but 8 waves per SIMD for rays given by the caller (their kernel waits on its
-// loads and on splines in LDS: 1e6 echelle rays 121 -> 112 us) and, where both
-// frames take an atomic of every ray and bound the trace, workgroups of 512
-// lanes from 2^20 rays on (1e7 echelle rays 926 -> 892 us; with fewer rays, or
-// one frame or none, 256 lanes are as fast or faster); and 1024 lanes and 8
-// waves per SIMD for recording traces with extents from 2^18 rays on, where
-// every workgroup has to meet the extremes before its rays lie inside them
-// (2^18 echelle rays 53 -> 47 us, 2^20 161 -> 123, 2^22 485 -> 401; 2^17 39 ->
-// 46, so not there).
-void trace_shape(const rt_hip_scheme* sch, bool gen, const TraceArgs& a, int rec, int& block, int& waves) {
-    block = sch->block;
-    waves = sch->waves;
-    if (sch->launch_given) return;
-    if (rec) {
-        if ((rec & rt::kRecExt) && a.n >= kExtRays) {
-            block = 1024;
-            waves = 8;
+struct LaunchShape {
+    int block, waves, mult;
+};
+
+// The launch of a trace (frames: into both frames).  The caller's holds for
+// every trace, the autotuner's for traces like those it timed: generated,
+// recording nothing, and with both frames or without as those were.  The
+// others take the defaults, but 8 waves per SIMD for rays given by the caller
+// (1e6 echelle rays into both frames 123 -> 120 us, 1e7 946 -> 935; with one
+// frame or none, with fewer rays and on the Czerny-Turner within 2% either
+// way); where both frames take an atomic of every ray and bound the trace,
+// workgroups of 512 lanes from 2^20 rays on (1e7 echelle rays of 2048
+// wavelengths 1014 -> 929 us, 4e6 410 -> 400; of 64 wavelengths within 2%,
+// the Czerny-Turner within 1%); and 1024 lanes and 8 waves per SIMD for
+// recording traces with extents from kExtRays on, where every workgroup has
+// to meet the extremes before its rays lie inside them (2^18 echelle rays 51
+// -> 46 us, 2^20 161 -> 123, 2^23 857 -> 763, 2^20 of the Czerny-Turner 51 ->
+// 42; 2^17 echelle rays 37 -> 45, so not there).
+LaunchShape launch_shape(const rt_hip_scheme* sch, bool gen, bool frames, int rec, uint64_t n) {
+    if (sch->launch_by == rt_hip_scheme::BY_CALLER ||
+        (sch->launch_by == rt_hip_scheme::BY_TUNER && gen && !rec && frames == sch->tuned_frames))
+        return LaunchShape{sch->block, sch->waves, sch->grid_mult};
+    LaunchShape l{kBlock, kDefaultWaves, kDefaultGridMult};
+    if (rec & rt::kRecExt) {
+        if (n >= kExtRays) {
+            l.block = 1024;
+            l.waves = 8;
         }
-        return;
+    } else if (!rec && !gen) {
+        l.waves = 8;
+    } else if (!rec && frames && n >= kFrameRays) {
+        l.block = 512;
     }
-    if (!gen) waves = 8;
-    const bool frames = (a.flags & RT_TRACE_HIST) && a.hist && (a.flags & RT_TRACE_FLUX) && a.flux;
-    if (gen && frames && a.n >= (1u << 20)) block = 512;
+    return l;
 }
 
 // The workgroups of a recording trace with extents: as many as are resident
@@ -1044,8 +1061,9 @@ int trace_launch(const rt_hip_scheme* sch, const double* beam_desc, uint64_t see
 
     const uint64_t nk = gen && sch->unroll ? dtab_nk(sch->dt, beam_desc) : 0;
     unsigned grid = 0;
-    int block, waves;
-    trace_shape(sch, gen, a, rec, block, waves);
+    const bool frames = (flags & RT_TRACE_HIST) && ccd_hist && (flags & RT_TRACE_FLUX) && ccd_flux;
+    const LaunchShape shape = launch_shape(sch, gen, frames, rec, n_rays);
+    const int block = shape.block, waves = shape.waves;
     // The workgroups of a recording trace with extents, and their rows of keys:
     // at least the rows that any size of the default launches takes, so that a
     // later call of another size finds its memory there, also while a graph is
@@ -1088,7 +1106,7 @@ int trace_launch(const rt_hip_scheme* sch, const double* beam_desc, uint64_t see
             resident < 1)
             resident = 1;
         uint64_t want = (n_rays + block - 1) / block;
-        uint64_t cap = (uint64_t)cus * resident * sch->grid_mult;
+        uint64_t cap = (uint64_t)cus * resident * shape.mult;
         grid = (unsigned)(want < cap ? want : cap);
         if (extents && (rc = ext_launch(want, (uint64_t)cus * resident)) != RT_OK) return rc;
         stats_target(a, sch->stat_copies, stats, grid);
@@ -1150,7 +1168,7 @@ extern "C" int rt_hip_trace_spots(const rt_hip_scheme* sch, const double* beam_d
     const uint64_t G = n_groups;
     // one partial row per tile of the launched kernel's workgroup size (the
     // generated kernel's or the generic one's): room for the smaller
-    const uint64_t b_min = (uint64_t)std::min(sch->block, kBlock);
+    const uint64_t b_min = (uint64_t)std::min(launch_shape(sch, true, false, rt::kRecSpots, n_rays).block, kBlock);
     const uint64_t tiles_max = (n_rays + b_min - 1) / b_min;
     if (tiles_max > (~0ull / 40) / G) return set_error(RT_ERR_BAD_VALUE, "too many rays x groups");
     rc = sch->work.ensure(WorkBufs::TRACE_PART, std::max<uint64_t>(tiles_max, 1) * G * 5 * sizeof(double));
@@ -1202,7 +1220,7 @@ extern "C" int rt_hip_scheme_set_launch(rt_hip_scheme* sch, int block, int waves
     sch->block = block;
     sch->waves = waves;
     sch->grid_mult = grid_mult;
-    sch->launch_given = true;
+    sch->launch_by = rt_hip_scheme::BY_CALLER;
     return RT_OK;
 }
 
@@ -1278,14 +1296,28 @@ extern "C" int rt_hip_autotune(rt_hip_scheme* sch, const double* beam_desc, uint
         (void)hipEventDestroy(e0);
         return set_error(RT_ERR_FAILED, "hipEventCreate");
     }
-    const int blocks[] = {128, 256};
+    // the launches of 128 and 256 lanes, and of as many lanes as an untuned trace
+    // of these rays takes where those are more (512, for large traces into both
+    // frames: the echelle's 1e7 rays 897 us, 942 with 256 lanes at best).  Of
+    // those the untuned trace's waves and the compiler's choice, grid multiples
+    // 8 and 16: 5 and 6 waves are within 0.5% of them, 8 waves and smaller
+    // multiples 3-6% slower, and every kernel takes 0.3 s to compile.
+    std::vector<int> blocks = {128, 256};
+    const bool frames = (flags & RT_TRACE_HIST) && hist.p && (flags & RT_TRACE_FLUX) && flux.p;
+    {
+        const auto by = sch->launch_by;
+        sch->launch_by = rt_hip_scheme::BY_RULE;
+        const int b = launch_shape(sch, true, frames, 0, n_sample).block;
+        sch->launch_by = by;
+        if (b > 256) blocks.push_back(b);
+    }
     const int wavess[] = {0, 5, 6, 7, 8};
     const int mults[] = {1, 2, 4, 8, 16};
     struct Cand { int b, w, m; float ms; int regs, local, u; };
     std::vector<Cand> cands;
     const int bb0 = sch->block, bw0 = sch->waves, bm0 = sch->grid_mult, bu0 = sch->unroll;
-    const bool given0 = sch->launch_given;
-    sch->launch_given = true;
+    const auto by0 = sch->launch_by;
+    sch->launch_by = rt_hip_scheme::BY_CALLER;
     // mean time of `reps` back-to-back launches of candidate c
     auto timed = [&](const Cand& c, int reps, float& ms) -> int {
         sch->block = c.b; sch->waves = c.w; sch->grid_mult = c.m; sch->unroll = c.u;
@@ -1316,6 +1348,7 @@ extern "C" int rt_hip_autotune(rt_hip_scheme* sch, const double* beam_desc, uint
         for (int w : wavess)
             for (int m : mults) {
                 if (rc != RT_OK || !rt_jit_enabled()) break;
+                if (b > 256 && (m < 8 || (w != 0 && w != kDefaultWaves))) continue;
                 Cand c{b, w, m, 1e30f, 0, 0, 1};
                 sch->block = b; sch->waves = w; sch->grid_mult = m;
                 if ((rc = run()) != RT_OK) break;
@@ -1394,7 +1427,12 @@ extern "C" int rt_hip_autotune(rt_hip_scheme* sch, const double* beam_desc, uint
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     sch->block = bb; sch->waves = bw; sch->grid_mult = bm; sch->unroll = bu;
-    if (rc != RT_OK) sch->launch_given = given0;
+    if (rc == RT_OK && best < 1e300) {
+        sch->launch_by = rt_hip_scheme::BY_TUNER;
+        sch->tuned_frames = frames;
+    } else {
+        sch->launch_by = by0;
+    }
     if (rc != RT_OK) return rc;
     if (best_ms) *best_ms = best;
     return RT_OK;
@@ -1412,7 +1450,7 @@ struct rt_hip_batch {
     double* tables_dev = nullptr;
     double* pool_dev = nullptr;
     uint64_t* ray_start_dev = nullptr;
-    int block = rt::kBlock, waves = 7, grid_mult = 16;   // as for one scheme
+    int block = rt::kBlock, waves = kDefaultWaves, grid_mult = kDefaultGridMult;   // as for one scheme
     int tiles_block = 0;             // workgroup size the tile arrays below are built for
     uint64_t n_tiles = 0;
     uint64_t* tile_start_dev = nullptr;

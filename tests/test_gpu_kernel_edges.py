@@ -241,6 +241,56 @@ def test_recording_captured_after_another_size(hip, first, then, block):
     ds.close()
 
 
+def test_tuned_launch_holds_for_traces_like_the_timed_ones(hip, monkeypatch, capfd):
+    """The launch of every trace as the library reports it: the tuner's for
+    generated traces with the frames it timed, the defaults of their kind for
+    the others, the caller's for all."""
+    from rt_amd import schemes
+    monkeypatch.setenv("RT_HIP_VERBOSE", "1")
+    n = 1 << 18
+    sc = schemes.czerny_turner(n, 1)
+    px = sc.detector().ccd["xdim"] * sc.detector().ccd["ydim"]
+    rays = torch.empty((7, n), dtype=torch.float64, device="cuda")
+    flag, loss = (torch.empty(n, dtype=d, device="cuda") for d in (torch.int8, torch.uint8))
+    ext = torch.zeros((sc.n_surf, hip.EXT_PER_SURF), dtype=torch.float64, device="cuda")
+    hist, flux = (torch.zeros(px, dtype=d, device="cuda") for d in (torch.int32, torch.float64))
+    gen, store, count = S.RT_TRACE_GENERATE, S.RT_TRACE_STORE, S.RT_TRACE_HIST
+    both = count | S.RT_TRACE_FLUX
+
+    def launches(ds):
+        calls = dict(generated=lambda: ds.trace(rays, flag, n=n, flags=gen | store | count, hist=hist),
+                     frames=lambda: ds.trace(rays, flag, n=n, flags=gen | store | both, hist=hist, flux=flux),
+                     given=lambda: ds.trace(rays, flag, n=n, flags=count, hist=hist),
+                     recorded=lambda: ds.trace_record(rays, flag, loss, extents=ext),
+                     few=lambda: ds.trace_record(rays, flag, loss, n=1000, extents=ext),
+                     spots=lambda: ds.trace_spots(1, n=n))
+        out = {}
+        for k, call in calls.items():
+            capfd.readouterr()
+            call()
+            torch.cuda.synchronize()
+            line = [v for v in capfd.readouterr().err.splitlines() if "generated kernel" in v][0]
+            out[k] = tuple(int(line.split(w)[1].split(",")[0]) for w in ("block ", "waves "))
+        return out
+    ds = hip.DeviceScheme(sc)
+    rules = dict(generated=(256, 7), frames=(256, 7), given=(256, 8), recorded=(1024, 8), few=(256, 7), spots=(256, 7))
+    assert launches(ds) == rules
+    ds.autotune(n_sample=20000, flags=store | count)
+    if ds.get_unroll():
+        assert launches(ds) == dict(rules, generated=ds.get_launch()[:2])
+    ds.set_unroll(True)
+    ds.set_launch(128, 5, 2)
+    assert set(launches(ds).values()) == {(128, 5)}
+    # a large sample into both frames: the launch that an untuned trace takes is
+    # among those timed
+    monkeypatch.setenv("RT_HIP_AUTOTUNE_LOG", "1")
+    for sample, there in ((1 << 20, True), ((1 << 20) - 1, False)):
+        capfd.readouterr()
+        ds.autotune(n_sample=sample, flags=both)
+        assert ("autotune: 512,7,16 " in capfd.readouterr().err) == there, sample
+    ds.close()
+
+
 def every_surface_kind():
     """a lens, a rotated auxiliary frame, a rotated stop, an aspheric and a
     toric lens, a plane lens face, both kinds of grating, a spherical and a
