@@ -187,7 +187,9 @@ struct AdjBufs {
 int adj_buffers(WorkBufs* w, size_t tape, size_t gacc, size_t part, const std::vector<int>& rows, bool upload_rows,
                 AdjBufs& out) {
     std::vector<int>& rows_key = w->params_key;
-    int rc = w->ensure(WorkBufs::TAPE, (tape + gacc + part) * sizeof(double));
+    int rc = w->ensure_together({{WorkBufs::TAPE, tape * sizeof(double)},
+                                 {WorkBufs::GACC, gacc * sizeof(double)},
+                                 {WorkBufs::PART, part * sizeof(double)}});
     if (rc != RT_OK) return rc;
     if (upload_rows && (rows != rows_key || !w->p[WorkBufs::PARAMS])) {
         rows_key.clear();
@@ -200,8 +202,8 @@ int adj_buffers(WorkBufs* w, size_t tape, size_t gacc, size_t part, const std::v
         rows_key = rows;
     }
     out.tape = w->get<double>(WorkBufs::TAPE);
-    out.gacc = out.tape + tape;
-    out.part = out.gacc + gacc;
+    out.gacc = w->get<double>(WorkBufs::GACC);
+    out.part = w->get<double>(WorkBufs::PART);
     out.params = w->get<int>(WorkBufs::PARAMS);
     return RT_OK;
 }

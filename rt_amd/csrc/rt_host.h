@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <initializer_list>
 #include <string>
 #include <vector>
 
@@ -26,7 +27,7 @@ int rt_set_error(int code, const char* fmt, ...) __attribute__((format(printf, 2
 // lives.  The calls of one owner share its buffers and therefore run in the
 // order of one stream.
 struct WorkBufs {
-    enum Slot { TAPE, PARAMS, SPOT_PART, SPOT_CS, DESCEND, EXT_KEYS, SAVE_HIST, SAVE_LPOS, SAVE_TILES,
+    enum Slot { TAPE, GACC, PART, PARAMS, SPOT_PART, SPOT_CS, DESCEND, EXT_KEYS, SAVE_HIST, SAVE_LPOS, SAVE_TILES,
                 SAVE_GPOS, TRACE_PART, N_SLOTS };
     void* p[N_SLOTS] = {};
     size_t have[N_SLOTS] = {};
@@ -35,6 +36,13 @@ struct WorkBufs {
     // p[s] holds at least `bytes` afterwards (RT_OK, or RT_ERR_BAD_ALLOC
     // with p[s] unchanged)
     int ensure(Slot s, size_t bytes);
+    // ensure() of every part, in one allocation where none of them has a buffer
+    // yet (a new scheme's first call); later each grows by itself
+    struct Part {
+        Slot slot;
+        size_t bytes;
+    };
+    int ensure_together(std::initializer_list<Part> parts);
     // p[s] is a new buffer of `bytes` afterwards (for contents that change
     // between calls while a captured graph may still read the old ones)
     int fresh(Slot s, size_t bytes);

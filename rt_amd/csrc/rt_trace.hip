@@ -64,6 +64,35 @@ int WorkBufs::ensure(Slot s, size_t bytes) {
     return fresh(s, std::max(bytes, have[s] + have[s] / 2));
 }
 
+int WorkBufs::ensure_together(std::initializer_list<Part> parts) {
+    size_t total = 0;
+    bool none = true;
+    for (const Part& q : parts) {
+        total += (q.bytes + 255) / 256 * 256;
+        none = none && !p[q.slot];
+    }
+    if (!none) {
+        for (const Part& q : parts) {
+            const int rc = ensure(q.slot, q.bytes);
+            if (rc != RT_OK) return rc;
+        }
+        return RT_OK;
+    }
+    void* base = nullptr;
+    if (hipMalloc(&base, total ? total : 8) != hipSuccess) {
+        (void)hipGetLastError();
+        return set_error(RT_ERR_BAD_ALLOC, "hipMalloc of %zu bytes of working memory failed", total);
+    }
+    owned.push_back(base);
+    char* at = (char*)base;
+    for (const Part& q : parts) {
+        p[q.slot] = at;
+        have[q.slot] = (q.bytes + 255) / 256 * 256;
+        at += have[q.slot];
+    }
+    return RT_OK;
+}
+
 int WorkBufs::fresh(Slot s, size_t want) {
     void* q = nullptr;
     if (hipMalloc(&q, want ? want : 8) != hipSuccess) {

@@ -291,6 +291,31 @@ def test_tuned_launch_holds_for_traces_like_the_timed_ones(hip, monkeypatch, cap
     ds.close()
 
 
+def test_more_parameters_do_not_take_a_second_tape(hip):
+    """A batched adjoint over more parameters than the one before needs more
+    partials, not another tape: the tape (hundreds of MB here) stays."""
+    from rt_amd import diff, schemes
+    sch = schemes.echelle(8, 16)
+    inst, _ = schemes.tolerance_instances(sch, 16, seed=1)
+    db = hip.DeviceBatch(inst, np.full(16, 30000))
+    pairs = [(p.surface, p.field) for p in diff.echelle_design_params(sch).params]
+    ps, pf = zip(*pairs)
+    seeds = torch.ones((16, 4, 3), dtype=torch.float64, device="cuda")
+    used = []
+    for m in (1, len(pairs)):
+        print(f"[adjoint memory] {m} parameters", flush=True)
+        grad = torch.zeros((16, m), dtype=torch.float64, device="cuda")
+        torch.cuda.synchronize()
+        before = torch.cuda.mem_get_info()[0]
+        db.adjoint(seeds, ps[:m], pf[:m], seed=3, grad=grad)
+        torch.cuda.synchronize()
+        used.append(before - torch.cuda.mem_get_info()[0])
+    db.close()
+    # 1,888 tiles of 256 lanes, tens of rows of 8 bytes each; the partials of 48
+    # parameters are 1,888 * 4 * 48 * 8 bytes = 2.9 MB
+    assert used[0] > 64 << 20 and used[1] < 32 << 20, used
+
+
 def every_surface_kind():
     """a lens, a rotated auxiliary frame, a rotated stop, an aspheric and a
     toric lens, a plane lens face, both kinds of grating, a spherical and a
