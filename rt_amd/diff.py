@@ -62,7 +62,7 @@ class ParamSpec:
         surfs = list(sch.surfaces)
         changed = {}
         for p, v in zip(self.params, values):
-            i = p.surface + len(surfs) if p.surface < 0 else p.surface
+            i = range(len(surfs))[p.surface]
             _set(surfs[i], p, float(v), changed.setdefault(i, {}))
         for i, fields in changed.items():
             surfs[i] = dataclasses.replace(surfs[i], **fields)
