@@ -234,6 +234,10 @@ def test_gpu_saved_beam_full_echelle(hip):
     rays, flag, loss, ext, perm, counts, out = gpu_saved(hip, sc, seed)
     rec = O.trace_record(sc, seed=seed, nthreads=16)
     assert np.array_equal(loss, rec.loss)
+    assert np.array_equal(np.isnan(ext), np.isnan(rec.extents))
+    on = ~np.isnan(ext)
+    floor = np.array([1.0, 1.0] + [length_scale(sc)] * 8 + [1.0, 1.0])[None, :].repeat(sc.n_surf, 0)
+    assert rel(ext[on], rec.extents[on], floor[on]) <= RTOL
     operm, ocounts = O.rearrange(rec.loss)
     assert np.array_equal(counts, ocounts)
     assert np.array_equal(perm, operm)
