@@ -461,7 +461,12 @@ int rt_hip_graph_destroy(rt_hip_graph *graph);
    RT_S_C, RT_S_K, RT_S_A + i, RT_S_CR, RT_S_DIST + j, RT_S_ANG + j (radians,
    the record's value) or RT_S_GRCONST (um) of a surface; grad (device,
    n_params) receives dLoss/dparameter, reduced in a fixed order.  Plane
-   gratings only.  No counterpart in the reference (it has no derivatives). */
+   gratings only.  A ray that cannot be differentiated (more than 8 Newton
+   iterations at a surface, a root of a discriminant that is zero there: a
+   refraction at the critical angle, an order that just leaves the grating) is
+   counted in RT_ST_ADJ_SKIP and adds nothing to that surface's derivatives
+   and those of the surfaces before it.  No counterpart in the reference (it
+   has no derivatives). */
 int rt_hip_adjoint(const rt_hip_scheme *scheme, const double *beam_desc, uint64_t seed, size_t n_rays,
                    const double *group_seeds, size_t n_groups, const int *param_surface,
                    const int *param_field, int n_params, double *grad, unsigned long long *stats,

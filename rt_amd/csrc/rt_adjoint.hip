@@ -264,9 +264,10 @@ void fill_beam(AdjArgs& a, const double* beam_desc) {
 }
 
 // minimum waves per SIMD asked of the generated kernels' register allocation:
-// 3 (168 VGPRs) measured fastest on the echelle's 48 parameters (a loss and its
-// gradient at 1e6 rays 360 us, 256 instances 12.1 ms; at 4, which spills 32
-// registers, 380 us and 13.3 ms); RT_HIP_ADJOINT_WAVES overrides (0: the
+// 3, where the echelle's 48 parameters take 144 VGPRs (batched 160) and nothing
+// spills (a loss and its gradient at 1e6 rays, back to back, 347 us, 256
+// instances 11.06 ms; at 2 the same within 0.3%, at 4, with 128 VGPRs and 18
+// LDS rows, 351 us and 11.11 ms); RT_HIP_ADJOINT_WAVES overrides (0: the
 // compiler's choice)
 int adjoint_waves() {
     const char* w = getenv("RT_HIP_ADJOINT_WAVES");

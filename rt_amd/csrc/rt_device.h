@@ -122,9 +122,10 @@ struct StatSurf {
 
 // ------------------------------------------------------------- FP64 math
 // The hardware estimates v_rcp_f64 and v_rsq_f64 (relative error below 5.3e-8
-// over 2.7e8 random arguments) refined to the FP64 rounding floor: one step of
-// third order, 1 + e + e^2 for the reciprocal and 1 + e/2 + 3e^2/8 for the
-// reciprocal square root, leaves e^3 < 2^-72 of the error.  Against two
+// over 2.7e8 random arguments) refined to the FP64 rounding floor by one step
+// of third order: 1 + e + e^2 for the reciprocal, with e = 1 - x r, leaves e^3
+// < 2^-72; 1 + e/2 + 3e^2/8 for the reciprocal square root, whose e = 1 - x y^2
+// is twice the estimate's error, leaves 5e^3/16 < 2^-71.  Against two
 // Newton-Raphson steps that is one instruction less per reciprocal and two
 // less per reciprocal square root, with the same largest errors over those
 // arguments (1.00 and 1.25 x 2^-53; quotient and square root equal the IEEE
@@ -587,8 +588,9 @@ __device__ __forceinline__ void asphere_pq(const SD& d, double r2, double& P, do
 // iteration evaluated at the point it returns, kept for the normal of the
 // action that follows (about 20 instructions a surface).  Conic: e the factor
 // of the normal, -dF/dX = e X; toric: f the profile F(Y), e its derivative.
-// The expressions are those of conic_derivs and toric_derivs, so the normal is
-// the same bit for bit.
+// The expressions are those of conic_derivs and toric_derivs without a given
+// profile (which the plugin's stages use), so the normal is the same bit for
+// bit.
 struct Profile {
     double e = 0.0, f = 0.0;
 };
@@ -970,7 +972,8 @@ __device__ __forceinline__ uint32_t trunc_u32(double v) {
     return u;
 }
 
-// v >= 0
+// v within 1e-9 of a whole number (a coordinate in (-1, 0), which truncates to
+// pixel 0, included: the fraction is v - floor(v))
 __device__ __forceinline__ bool near_edge(double v) {
     const double f = __builtin_amdgcn_fract(v);
     return (f < 1e-9) | (1.0 - f < 1e-9);

@@ -1005,7 +1005,8 @@ struct LaunchShape {
 // recording traces with extents from kExtRays on, where every workgroup has
 // to meet the extremes before its rays lie inside them (2^18 echelle rays 51
 // -> 46 us, 2^20 161 -> 123, 2^23 857 -> 763, 2^20 of the Czerny-Turner 51 ->
-// 42; 2^17 echelle rays 37 -> 45, so not there).
+// 42; 2^17 echelle rays 37 -> 45, so not there; with 4 waves, where the
+// echelle's kernel does not spill its 52 bytes a lane, 2^20 130, 2^23 855).
 LaunchShape launch_shape(const rt_hip_scheme* sch, bool gen, bool frames, int rec, uint64_t n) {
     if (sch->launch_by == rt_hip_scheme::BY_CALLER ||
         (sch->launch_by == rt_hip_scheme::BY_TUNER && gen && !rec && frames == sch->tuned_frames))
