@@ -546,9 +546,9 @@ struct rt_hip_scheme {
     std::vector<double> dpool;       // device spline records
     // launch of the generated kernel (rt_hip_scheme_set_launch, rt_hip_autotune)
     // (default 256 lanes, 7 waves/SIMD, 16 workgroups per resident slot: the
-    // autotuner's usual choice on the echelle, and the fastest of a sweep of
-    // the batched trace over 1024 instances of uneven size, 21.3 ms against
-    // 23.7-24.0 ms at a grid multiple of 2)
+    // fastest of a sweep of the batched trace over 1024 instances of uneven
+    // size, 21.3 ms against 23.7-24.0 ms at a grid multiple of 2; launch_shape
+    // says which traces of one scheme take another)
     int block = rt::kBlock;          // lanes per workgroup
     int waves = kDefaultWaves;       // minimum waves per SIMD asked of the compiler (0: its choice)
     int grid_mult = kDefaultGridMult;    // persistent workgroups per CU = grid_mult x resident ones

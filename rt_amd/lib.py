@@ -254,6 +254,7 @@ class DeviceScheme:
         return bool(u.value)
 
     def get_launch(self):
+        """The launch that was set or tuned, else the default (rt_hip_scheme_get_launch)."""
         b, w, m = C.c_int(), C.c_int(), C.c_int()
         check(lib().rt_hip_scheme_get_launch(self.handle, C.byref(b), C.byref(w), C.byref(m)),
               "rt_hip_scheme_get_launch")
@@ -261,7 +262,8 @@ class DeviceScheme:
 
     def autotune(self, n_sample: int, flags: int, seed: int = 0, beam=None, stream=None) -> float:
         """Time the candidate launches on n_sample generated rays and keep the
-        fastest (rt_hip_autotune); returns its time in ms."""
+        fastest for generated traces with the same frames, both or not both
+        (rt_hip_autotune); returns its time in ms."""
         import torch
         b = np.ascontiguousarray((beam if beam is not None else self.scheme.beam).pack())
         if stream is None:
